@@ -306,8 +306,8 @@ int rta_trace_cis(const rta_triangle *tris, int n_tris, const rta_node *nodes,
  * tri4 (3 float4 per triangle: a, a-b, a-c with the same float values
  * intersect_tri_opt forms; the w of a leaf's last triangle is nonzero).
  * flags (device word): bit 0 set when some box coordinate is outside the
- * range where the division-free slab test is exact (then the traversal
- * uses IEEE divisions for every ray). */
+ * range where the division-free slab test is exact, or some box has a min
+ * above its max (then the traversal uses IEEE divisions for every ray). */
 int rta_bvh_pack(rta_node_pair *pairs, float *tri4, uint32_t *flags,
                  const rta_node *nodes, int n_nodes,
                  const rta_triangle *tris, int n_tris, rta_stream s);

@@ -142,18 +142,25 @@ __device__ inline bool box_test(float lo_x, float lo_y, float lo_z,
 //    values do.
 // Hence (hit, dist) equal box_test's whenever every quotient is exact:
 // coord_fast_ok boxes and origins, ray_nz_ok directions.
+__device__ inline void box_slabs(float lo_x, float lo_y, float lo_z,
+                                 float hi_x, float hi_y, float hi_z,
+                                 float ox, float oy, float oz,
+                                 float dx, float dy, float dz,
+                                 float yx, float yy, float yz, float &tn, float &tf) {
+	const float ax = div_cr1(lo_x - ox, dx, yx), bx = div_cr1(hi_x - ox, dx, yx);
+	const float ay = div_cr1(lo_y - oy, dy, yy), by = div_cr1(hi_y - oy, dy, yy);
+	const float az = div_cr1(lo_z - oz, dz, yz), bz = div_cr1(hi_z - oz, dz, yz);
+	tn = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fminf(az, bz));
+	tf = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz));
+}
 __device__ inline bool box_test_nz(float lo_x, float lo_y, float lo_z,
                                    float hi_x, float hi_y, float hi_z,
                                    float ox, float oy, float oz,
                                    float dx, float dy, float dz,
                                    float yx, float yy, float yz, float &dist) {
-	const float ax = div_cr1(lo_x - ox, dx, yx), bx = div_cr1(hi_x - ox, dx, yx);
-	const float ay = div_cr1(lo_y - oy, dy, yy), by = div_cr1(hi_y - oy, dy, yy);
-	const float az = div_cr1(lo_z - oz, dz, yz), bz = div_cr1(hi_z - oz, dz, yz);
-	const float tn = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fminf(az, bz));
-	const float tf = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz));
-	dist = tn;
-	return tn <= tf && tf >= 0.0f;
+	float tf;
+	box_slabs(lo_x, lo_y, lo_z, hi_x, hi_y, hi_z, ox, oy, oz, dx, dy, dz, yx, yy, yz, dist, tf);
+	return dist <= tf && tf >= 0.0f;
 }
 
 // A coordinate is "fast-safe" if it is 0 or 2^-73 <= |x| <= 2^59.  For two

@@ -12,6 +12,7 @@
 #include "internal.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace rta_hip {
 
@@ -179,14 +180,17 @@ __device__ inline void mark_leaf_end(float4 *tri4, const rta_node &leaf) {
 	tri4[3 * last].w = __uint_as_float(1u);
 }
 
+// ordered, too: the traversal's staged fetch takes an axis's near plane by
+// the direction's sign, where the reference swaps the two quotients
 __device__ inline bool box_fast_ok(const rta_aabb &b) {
 	return coord_fast_ok(b.min.x) && coord_fast_ok(b.min.y) && coord_fast_ok(b.min.z) &&
-	       coord_fast_ok(b.max.x) && coord_fast_ok(b.max.y) && coord_fast_ok(b.max.z);
+	       coord_fast_ok(b.max.x) && coord_fast_ok(b.max.y) && coord_fast_ok(b.max.z) &&
+	       b.min.x <= b.max.x && b.min.y <= b.max.y && b.min.z <= b.max.z;
 }
 
 // One pair record per inner node; flags bit 0 is set when some tested box
-// has a coordinate outside the fast-safe range (then every ray uses the
-// IEEE division path).
+// has a coordinate outside the fast-safe range or a min above its max (then
+// every ray uses the IEEE division path).
 __device__ inline void pack_pair(rta_node_pair *__restrict__ pairs, float4 *__restrict__ tri4,
                                  uint32_t *__restrict__ flags, const rta_node *__restrict__ nodes,
                                  int x);
@@ -619,6 +623,16 @@ __global__ void fill_queue_kernel(uint32_t *queue) {
 // sentinel back with t = FLT_MAX, kernels.cu:793-794,853).  ANY_HIT as in
 // trace_cis_packed_kernel.
 //
+// What bounds it: incoherent rays (diffuse bounces) the vector memory path,
+// whose cost is lines touched per load instruction and lane -- 42 active
+// lanes each fetching its own 64-byte record in four loads -- hence the
+// staged fetch in `run` below; coherent rays the VALU (about 95
+// instructions per wave-step at inner nodes, 116 before the stack's top
+// moved to a register, the decision's masks to scalar registers and the
+// records' stores out of the step).  On the 2.3 M-triangle terrain, 2.07 M
+// rays each: bounce rays 1,917 -> 1,582 us, primary rays 1,826-1,886 ->
+// 1,634 us; shadow rays of a 400 k-triangle terrain (0.88 M) 739 -> 632 us.
+//
 // BATCHED: rays of many meshes in one launch.  Ray r belongs to the mesh
 // whose [ray_off, ray_off + n_rays) holds it; that mesh's pair records start
 // at pairs[node_off], its tri4 records at tri4[3 * tri_off], its flag word
@@ -638,6 +652,39 @@ struct SeedArgs {
 	const int32_t *top = nullptr;
 };
 
+// A lane without a ray holds kIdle as its current word, which no node or
+// leaf has (an even word is a leaf's first triangle << 1, and a mesh has
+// fewer than 2^31 - 1 triangles); the same word marks the stack's bottom.
+constexpr uint32_t kIdle = 0xfffffffeu;
+constexpr uint32_t kNoRay = 0xffffffffu;
+typedef float Pair __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) uint32_t LdsWord;
+typedef __attribute__((address_space(3))) char LdsByte;
+typedef __attribute__((address_space(3))) Pair LdsPair;
+typedef __attribute__((address_space(1))) char GlobalByte;
+// Stack rows in LDS, and how many of them move to private memory at once.
+// With the 4 KiB stage, 11 + 3 rows make 7,680 B per wave, six of the 1,280-B
+// units LDS is handed out in: 20 resident waves per CU, where 13 rows leave
+// 18 (primary rays 1,634 against 1,688 us, bounce rays 1,582 against 1,602 us
+// per 2.07 M on the 2.3 M-triangle terrain); 9 rows spill more and gain no
+// wave (1,659 / 1,607 us).
+constexpr int kRows = 11, kSpill = 5;
+// At least this many lanes whose neighbour stands at another inner node make
+// a wave take its next round of steps through the stage.  Of thresholds 12,
+// 24, 36 and never: primary rays 1,793 / 1,698 / 1,683 / 1,603 us, bounce
+// rays 1,617 / 1,613 / 1,609 / 2,141 us (16 rows, same scene).
+constexpr int kStageMin = 36;
+
+// The largest x with x < ct && x <= tmax, for ct > 0 (-inf for a NaN tmax,
+// which accepts nothing).
+__device__ inline float accept_limit(float ct, float tmax) {
+	const float below = __uint_as_float(__float_as_uint(ct) - 1u);
+	return tmax == tmax ? fminf(below, tmax) : -__builtin_inff();
+}
+
+__device__ inline uint64_t lanes(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+__device__ inline bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
 // STACK: the LDS stack's entries (kStack, or fewer for a smaller LDS
 // footprint and so more resident waves).  With STACK < kStack a ray that
 // would push beyond it is abandoned and appended to the overflow list ovf
@@ -645,7 +692,7 @@ struct SeedArgs {
 // with kStack entries.  ray_list (optional): trace the rays ray_list[1 ..
 // ray_list[0]] instead of 0 .. n-1.
 template <int BLOCK, bool ANY_HIT, bool BATCHED, bool SEEDED = false, int STACK = kStack>
-__global__ __launch_bounds__(BLOCK) void trace_cis_persistent_kernel(
+__global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
     const float4 *__restrict__ tri4, const float4 *__restrict__ pairs,
     const uint32_t *__restrict__ flags, uint32_t root_word, const float *__restrict__ ro,
     const float *__restrict__ rd, const float *__restrict__ rmax, int n_rays,
@@ -655,8 +702,21 @@ __global__ __launch_bounds__(BLOCK) void trace_cis_persistent_kernel(
     const uint32_t *__restrict__ root_words, uint32_t *__restrict__ ovf,
     const uint32_t *__restrict__ ray_list, SeedArgs seed) {
 	static_assert(!SEEDED || (!ANY_HIT && !BATCHED), "seeding: closest hit on one mesh");
-	static_assert(STACK <= kStack, "at most kStack entries");
-	__shared__ uint32_t stack[STACK][BLOCK];
+	static_assert(STACK >= kRows && STACK <= kStack, "kRows to kStack entries");
+	// Row r of the stack holds one word per lane.  The top entry lives in a
+	// register (`top`), the ones below it in rows 1 .. kRows, the lowest of
+	// them the bottom mark kIdle; `sp` points at the last of those rows (row
+	// 0 while there is none).  Row 0 is read, and its value dropped, when a
+	// lane pops the mark (sp is row -1 from then on, and the idle lane may
+	// still read it); row kRows + 1 is written when a lane whose rows are
+	// full takes a step.  A push beyond kRows first moves the lowest kSpill
+	// rows (or what is left of STACK) to private memory, `deep`, of which
+	// `spilled` entries are in use.
+	__shared__ uint32_t stack[(kRows + 3) * BLOCK];
+	__shared__ float4 stage[BLOCK / kWave][4][kWave];   // see run
+	constexpr int kDeep = STACK - kRows;
+	uint32_t deep[kDeep + kSpill];
+	int spilled = 0;
 	const int lt = threadIdx.x;
 	const int lane = __lane_id();
 	const uint64_t lower = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -670,14 +730,26 @@ __global__ __launch_bounds__(BLOCK) void trace_cis_persistent_kernel(
 	const uint32_t n_treelets = SEEDED ? *seed.count : 0u;
 	bool seeding = false;   // SEEDED: the lane is in its treelet phase
 
-	bool active = false, exhausted = false;
-	uint32_t ray = 0, curr = 0;
+	LdsWord *bottom = (LdsWord *)&stack[BLOCK + lt];
+	asm("" : "+v"(bottom));   // one register, not lane base + offset
+	LdsWord *const limit = bottom + kRows * BLOCK;
+	LdsWord *sp = bottom;
+	const int wave = __builtin_amdgcn_readfirstlane(lt / kWave);
+	const int quad = lane & 3;
+	// byte b (a multiple of 8) of this lane's record in the stage
+	LdsByte *const record = (LdsByte *)&stage[wave][quad][lane & ~3];
+	auto staged = [&](int b) { return (const LdsPair *)(record + ((((b >> 4) ^ quad) << 4) | (b & 8))); };
+
+	uint32_t curr = kIdle, top = kIdle, ray = kNoRay;
+	bool exhausted = false;
 	uint32_t node_base = 0, tri_base = 0;
-	int sp = -1;
 	float ox = 0, oy = 0, oz = 0, dx = 0, dy = 0, dz = 0, yx = 0, yy = 0, yz = 0, tmax = 0;
-	float ct = FLT_MAX, cb = 0, cg = 0;
+	// lim: the largest entry distance or hit distance still accepted,
+	// min(tmax, the float below ct), so that `x <= lim` is the reference's
+	// x < closest.t && x <= max_t
+	float ct = FLT_MAX, cb = 0, cg = 0, lim = 0;
 	uint32_t cref = 0;
-	bool fast = false;
+	bool fast = true;
 	// Rounds (of at most `steps` wave-steps) since the last refill.  Every
 	// wave-step advances at least one lane and each lane holds at most one
 	// ray per refill, so with a valid tree (at most 2 * nodes < kMaxSteps
@@ -686,30 +758,237 @@ __global__ __launch_bounds__(BLOCK) void trace_cis_persistent_kernel(
 	// in an error count per active ray instead of an endless loop.
 	uint64_t rounds = 0;
 	const uint64_t round_limit = 64ull * kMaxSteps / (uint64_t)steps + 2;
-	// write the ray's record (hits[ray].t = FLT_MAX alone on a miss) and
-	// free the lane
-	auto finish = [&]() {
-		if (ct != FLT_MAX) {
-			rta_hit hres;
-			hres.t = ct; hres.beta = cb; hres.gamma = cg; hres.ref = cref;
-			hits[ray] = hres;
-		} else {
-			hits[ray].t = FLT_MAX;
+	uint64_t slow_lanes = 0;   // lanes whose ray takes the IEEE box test
+	uint64_t deep_lanes = 0;   // lanes with spilled stack entries
+
+	// The reference's decision at an inner node (kernels.cu:818-835) for the
+	// lanes there, without branches: both children kept -> enter the nearer,
+	// the left one on a tie, and push the other; one kept -> enter it; none ->
+	// pop (the bottom mark makes the lane idle).  (dl, fl), (dr, fr): the
+	// children's entry and exit distances; wl, wr: their words; below: the
+	// entry below the top, whose own row the caller has written.
+	auto decide = [&](float dl, float fl, float dr, float fr, uint32_t wl, uint32_t wr,
+	                  uint32_t below) {
+		// lane masks in scalar registers
+		uint64_t hl = lanes(dl <= fl) & lanes(dl <= lim) & lanes(fl >= 0.0f);
+		uint64_t hr = lanes(dr <= fr) & lanes(dr <= lim) & lanes(fr >= 0.0f);
+		if (slow_lanes != 0ull) {
+			bool sl = false, sr = false;
+			if (!fast) {
+				const float4 *p = pairs + 4 * ((size_t)node_base + (curr >> 1));
+				const float4 q0 = p[0], q1 = p[1], q2 = p[2];
+				sl = box_test(q0.x, q0.z, q1.x, q1.z, q2.x, q2.z, ox, oy, oz, dx, dy, dz, dl);
+				sr = box_test(q0.y, q0.w, q1.y, q1.w, q2.y, q2.w, ox, oy, oz, dx, dy, dz, dr);
+			}
+			hl = (hl & ~slow_lanes) | (lanes(sl) & lanes(dl <= lim));
+			hr = (hr & ~slow_lanes) | (lanes(sr) & lanes(dr <= lim));
 		}
-		active = false;
+		const uint64_t both = hl & hr;
+		const bool any = in_mask(hl | hr), push = in_mask(both);
+		const bool enter_left = in_mask(hl & (lanes(dl <= dr) | ~hr));
+		const uint32_t near_w = enter_left ? wl : wr, far_w = enter_left ? wr : wl;
+		curr = any ? near_w : top;
+		top = push ? far_w : (any ? top : below);
+		const uint64_t over = both & lanes(sp == limit);
+		if (over != 0ull) {
+			if (in_mask(over)) {
+				if (spilled < kDeep) {
+					const int m = min(kSpill, kDeep - spilled);
+#pragma nounroll
+					for (int i = 0; i < m; ++i) deep[spilled + i] = bottom[(1 + i) * BLOCK];
+#pragma nounroll
+					for (int i = 1; i <= kRows + 1 - m; ++i) bottom[i * BLOCK] = bottom[(i + m) * BLOCK];
+					sp -= m * BLOCK;
+					spilled += m;
+				} else {
+					// a push beyond STACK entries ends the ray with an error count
+					// (STACK = kStack) or on the overflow list (STACK < kStack)
+					curr = kIdle;
+					sp = bottom - BLOCK;
+					if (STACK < kStack) {
+						ovf[1 + atomicAdd(ovf, 1u)] = ray;   // traced again
+						ray = kNoRay;
+					} else {
+						atomicAdd(err, 1u);
+					}
+				}
+			}
+			deep_lanes |= lanes(spilled != 0);
+		}
+		sp += push ? BLOCK : (any ? 0 : -BLOCK);
+	};
+
+	// Up to `steps` wave-steps.  Each is an inner-node step or a leaf step
+	// for the whole wave.  GATHER: at an inner node every lane loads its own
+	// node's record, four 16-byte loads of which each touches another line
+	// per lane.  Otherwise the four lanes of a quad load the record of one of
+	// them together, in four rounds straight into LDS (round k: the node of
+	// lane 4j + k), so that a round asks for 16 whole records instead of a
+	// quarter of 64.  Round k keeps quarter q of a record in slot q ^ k: the
+	// reads below then meet no bank conflicts.  From LDS a lane reads each
+	// axis's near and far planes by the sign of its direction; where the
+	// division-free test is allowed lo <= hi, and div_cr1 is correctly
+	// rounded, hence monotonic, so these give the minimum and the maximum of
+	// the axis's two quotients.
+	auto run = [&](auto gather) {
+		constexpr bool GATHER = decltype(gather)::value;
+		const LdsPair *anx = nullptr, *any_ = nullptr, *anz = nullptr, *afx = nullptr,
+		              *afy = nullptr, *afz = nullptr;
+		uint32_t quarter[4] = {};   // the record's bytes this lane loads in round k
+		if (!GATHER) {
+			for (int k = 0; k < 4; ++k) quarter[k] = (uint32_t)((quad ^ k) << 4);
+			anx = staged(dx < 0.0f ? 24 : 0);
+			afx = staged(dx < 0.0f ? 0 : 24);
+			any_ = staged(dy < 0.0f ? 32 : 8);
+			afy = staged(dy < 0.0f ? 8 : 32);
+			anz = staged(dz < 0.0f ? 40 : 16);
+			afz = staged(dz < 0.0f ? 16 : 40);
+		}
+		for (int k = 0; k < steps; ++k) {
+			const uint64_t act = lanes(curr != kIdle);
+			if (act == 0ull) break;
+			const uint64_t inner_lanes = lanes((curr & 1u) != 0u);
+			// Wave-uniform choice of this step's kind: a leaf step once
+			// leaf_min of 64 lanes, scaled to the lanes still active, wait at
+			// leaves (a draining wave does not hold its last rays there).
+			const int n_act = __popcll(act);
+			const int n_leaf = n_act - __popcll(inner_lanes);
+			const int thr = (n_act * leaf_min + 63) >> 6;
+			if (inner_lanes != 0ull && n_leaf < thr) {
+				if (GATHER) {
+					if (curr & 1u) {
+						// the entry below the top, needed if this step pops, and the
+						// top's own row, needed if it pushes: off the path that
+						// waits for the loads
+						const uint32_t below = sp[0];
+						sp[BLOCK] = top;
+						const float4 *p = pairs + 4 * ((size_t)node_base + (curr >> 1));
+						const float4 q0 = p[0], q1 = p[1], q2 = p[2];
+						const uint2 words = *reinterpret_cast<const uint2 *>(p + 3);
+						float dl, dr, fl, fr;
+						box_slabs(q0.x, q0.z, q1.x, q1.z, q2.x, q2.z, ox, oy, oz, dx, dy, dz, yx, yy,
+						          yz, dl, fl);
+						box_slabs(q0.y, q0.w, q1.y, q1.w, q2.y, q2.w, ox, oy, oz, dx, dy, dz, yx, yy,
+						          yz, dr, fr);
+						decide(dl, fl, dr, fr, words.x, words.y, below);
+					}
+				} else {
+					const uint32_t below = sp[0];
+					sp[BLOCK] = top;
+					// lanes not at an inner node ask for record 0
+					const uint32_t id = (curr & 1u) ? node_base + (curr >> 1) : 0u;
+					const uint64_t addr = (uint64_t)(uintptr_t)pairs + ((uint64_t)id << 6);
+					const int addr_lo = (int)(uint32_t)addr, addr_hi = (int)(uint32_t)(addr >> 32);
+#define RTA_ROUND(K)                                                                                \
+	{                                                                                               \
+		const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, addr_lo, (K) * 0x55, 0xf, 0xf, true) | \
+		                    quarter[K];                                                             \
+		const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, addr_hi, (K) * 0x55, 0xf, 0xf, true); \
+		__builtin_amdgcn_global_load_lds((const GlobalByte *)(((uint64_t)hi << 32) | lo),           \
+		                                 (LdsByte *)&stage[wave][K][0], 16, 0, 0);                  \
+	}
+					RTA_ROUND(0) RTA_ROUND(1) RTA_ROUND(2) RTA_ROUND(3)
+#undef RTA_ROUND
+					// the stage is this wave's own: its loads are waited for, no
+					// barrier
+					asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+					if (curr & 1u) {
+						const Pair nx = *anx, ny = *any_, nz = *anz, fx = *afx, fy = *afy, fz = *afz;
+						const Pair words = *staged(48);
+						auto slabs = [&](int c, float &tn, float &tf) {
+							tn = fmaxf(fmaxf(div_cr1(nx[c] - ox, dx, yx), div_cr1(ny[c] - oy, dy, yy)),
+							           div_cr1(nz[c] - oz, dz, yz));
+							tf = fminf(fminf(div_cr1(fx[c] - ox, dx, yx), div_cr1(fy[c] - oy, dy, yy)),
+							           div_cr1(fz[c] - oz, dz, yz));
+						};
+						float dl, dr, fl, fr;
+						slabs(0, dl, fl);
+						slabs(1, dr, fr);
+						decide(dl, fl, dr, fr, __float_as_uint(words[0]), __float_as_uint(words[1]),
+						       below);
+					}
+				}
+			} else if (!(curr & 1u) && curr != kIdle) {
+				uint32_t i = curr >> 1;
+				const float4 *tb = tri4 + 3 * (size_t)tri_base;
+				// pop; a shadow ray ends at its first hit, a treelet phase at
+				// its first hit leaf (any real hit is a valid bound)
+				curr = top;
+				top = *sp;
+				sp -= BLOCK;
+				while (true) {
+					const float4 v0 = tb[3 * (size_t)i + 0];
+					const float4 v1 = tb[3 * (size_t)i + 1];
+					const float4 v2 = tb[3 * (size_t)i + 2];
+					float t, be, ga;
+					if (tri_test(v0.x, v0.y, v0.z, v1.x, v1.y, v1.z, v2.x, v2.y, v2.z, ox, oy, oz,
+					             dx, dy, dz, t, be, ga)) {
+						if (t <= lim) {
+							ct = t; cb = be; cg = ga; cref = i;
+							lim = accept_limit(t, tmax);
+							if (ANY_HIT) {
+								curr = kIdle;
+								break;
+							}
+							if (SEEDED && seeding) curr = kIdle;
+						}
+					}
+					if (__float_as_uint(v0.w) != 0u) break;
+					++i;
+				}
+			}
+			if (deep_lanes != 0ull) {
+				// a lane that used up its rows takes back its last spilled entries
+				if (spilled != 0 && sp == bottom && curr != kIdle) {
+					const int part = spilled % kSpill, m = part ? part : kSpill;
+					spilled -= m;
+#pragma nounroll
+					for (int i = 0; i < m; ++i) bottom[(1 + i) * BLOCK] = deep[spilled + i];
+					sp += m * BLOCK;
+				}
+				deep_lanes = lanes(spilled != 0);
+			}
+			if (SEEDED && seeding && curr == kIdle) {
+				// the treelet phase ends: its closest t (a real hit, or
+				// FLT_MAX), widened by seed_bound's margin, bounds the
+				// traversal of the whole tree
+				tmax = fminf(tmax, seed_bound(ct));
+				ct = FLT_MAX;
+				lim = accept_limit(ct, tmax);
+				curr = root_word;
+				top = kIdle;
+				sp = bottom;
+				spilled = 0;
+				seeding = false;
+			}
+		}
 	};
 
 	while (true) {
-		const uint64_t idle = __ballot(!active);
+		const uint64_t idle = lanes(curr == kIdle);
 		const int nidle = __popcll(idle);
-		if (!exhausted && nidle >= refill_min) {
+		if (nidle == kWave || (!exhausted && nidle >= refill_min)) {
+			// write the finished rays' records (t = FLT_MAX alone on a miss)
+			if (curr == kIdle && ray != kNoRay) {
+				if (ct != FLT_MAX) {
+					rta_hit hres;
+					hres.t = ct; hres.beta = cb; hres.gamma = cg; hres.ref = cref;
+					hits[ray] = hres;
+				} else {
+					hits[ray].t = FLT_MAX;
+				}
+				ray = kNoRay;
+			}
+			if (exhausted) break;   // and every lane is idle
 			rounds = 0;
 			const int leader = __ffsll((unsigned long long)idle) - 1;
 			uint32_t base = 0;
 			if (lane == leader) base = atomicAdd(queue, (uint32_t)nidle);
-			base = __shfl(base, leader);
+			// readlane, not a shuffle: the result is wave-uniform for the
+			// compiler too, and with it the loop's control flow
+			base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);
 			if (base + (uint32_t)nidle >= n) exhausted = true;
-			if (!active) {
+			if (curr == kIdle) {
 				const uint32_t my = base + (uint32_t)__popcll(idle & lower);
 				if (my < n) {
 					ray = ray_list ? ray_list[1 + my] : my;
@@ -748,108 +1027,31 @@ __global__ __launch_bounds__(BLOCK) void trace_cis_persistent_kernel(
 					}
 					yx = 1.0f / dx; yy = 1.0f / dy; yz = 1.0f / dz;
 					ct = FLT_MAX;
-					sp = -1;
-					active = true;
+					lim = accept_limit(ct, tmax);
+					top = kIdle;
+					sp = bottom;
+					spilled = 0;
 				}
 			}
+			slow_lanes = lanes(curr != kIdle && !fast);
+			deep_lanes = lanes(spilled != 0);
+			if (lanes(curr != kIdle) == 0ull) break;   // the queue was empty
 		}
-		// with refill_min <= 64 an all-idle wave has just refilled, so an
-		// all-idle wave here means the queue is exhausted
-		if (__ballot(active) == 0ull) break;
 		if (++rounds > round_limit) {
 			// malformed tree: every active ray ends with an error count
-			if (active) {
+			if (curr != kIdle) {
 				atomicAdd(err, 1u);
-				finish();
+				curr = kIdle;
 			}
 			continue;
 		}
-		for (int k = 0; k < steps; ++k) {
-			const bool is_inner = (curr & 1u) != 0u;
-			const uint64_t act = __ballot(active);
-			if (act == 0ull) break;
-			const uint64_t inner_lanes = __ballot(active && is_inner);
-			// Wave-uniform choice of this step's kind: a leaf step once
-			// leaf_min of 64 lanes, scaled to the lanes still active, wait at
-			// leaves (a draining wave does not hold its last rays there).
-			const int n_leaf = __popcll(act & ~inner_lanes);
-			const int thr = (__popcll(act) * leaf_min + 63) >> 6;
-			const bool leaf_step = inner_lanes == 0ull || n_leaf >= thr;
-			if (!active || is_inner == leaf_step) continue;
-			bool done, overflow = false;
-			if (!leaf_step) {
-				const float4 *p = pairs + 4 * ((size_t)node_base + (curr >> 1));
-				const float4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3];
-				float dl, dr;
-				bool hl, hr;
-				pair_boxes(q0, q1, q2, fast, ox, oy, oz, dx, dy, dz, yx, yy, yz, hl, dl, hr, dr);
-				hl = hl && dl < ct && dl <= tmax;
-				hr = hr && dr < ct && dr <= tmax;
-				const uint32_t wl = __float_as_uint(q3.x), wr = __float_as_uint(q3.y);
-				// The reference's decision (kernels.cu:818-835) without
-				// branches: both kept -> enter the nearer, the left one on a
-				// tie, and push the other; one kept -> enter it; none -> pop,
-				// or finish on an empty stack.  The far child is written one
-				// slot above the top on every step (after the top is read);
-				// only a push makes that slot part of the stack.  On a full
-				// stack (STACK entries) there is no slot above the top: the
-				// top entry is written back with its own value, so a step that
-				// keeps one child or none leaves the stack intact, and a push
-				// ends the ray with an error count (STACK = kStack) or on the
-				// overflow list (STACK < kStack).
-				const bool both = hl && hr, any = hl || hr;
-				const bool enter_left = both ? (dl <= dr) : hl;
-				const bool full = sp + 1 >= STACK;
-				const uint32_t popped = stack[sp >= 0 ? sp : 0][lt];
-				stack[full ? STACK - 1 : sp + 1][lt] = full ? popped : (enter_left ? wr : wl);
-				curr = any ? (enter_left ? wl : wr) : popped;
-				overflow = both && full;
-				done = overflow || (!any && sp < 0);
-				sp += both ? 1 : (any ? 0 : -1);
-			} else {
-				uint32_t i = curr >> 1;
-				const float4 *tb = tri4 + 3 * (size_t)tri_base;
-				while (true) {
-					const float4 v0 = tb[3 * (size_t)i + 0];
-					const float4 v1 = tb[3 * (size_t)i + 1];
-					const float4 v2 = tb[3 * (size_t)i + 2];
-					float t, be, ga;
-					if (tri_test(v0.x, v0.y, v0.z, v1.x, v1.y, v1.z, v2.x, v2.y, v2.z, ox, oy, oz,
-					             dx, dy, dz, t, be, ga)) {
-						if (t < ct && t <= tmax) {
-							ct = t; cb = be; cg = ga; cref = i;
-							if (ANY_HIT) break;
-						}
-					}
-					if (__float_as_uint(v0.w) != 0u) break;
-					++i;
-				}
-				// pop, or finish (empty stack, a shadow ray's first hit, or the
-				// end of a treelet phase at its first hit leaf: any real hit
-				// is a valid bound)
-				curr = stack[sp >= 0 ? sp : 0][lt];
-				done = (ANY_HIT && ct != FLT_MAX) || (SEEDED && seeding && ct != FLT_MAX) || sp < 0;
-				--sp;
-			}
-			if (done) {
-				if (overflow) {
-					if (STACK < kStack) ovf[1 + atomicAdd(ovf, 1u)] = ray;   // traced again
-					else atomicAdd(err, 1u);
-				}
-				if (SEEDED && seeding) {
-					// the treelet phase ends: its closest t (a real hit, or
-					// FLT_MAX), widened by seed_bound's margin, bounds the
-					// traversal of the whole tree
-					tmax = fminf(tmax, seed_bound(ct));
-					ct = FLT_MAX;
-					curr = root_word;
-					sp = -1;
-					seeding = false;
-				} else {
-					finish();
-				}
-			}
-		}
+		// Lanes whose neighbour stands at another node: coherent waves gather
+		const uint32_t beside = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)curr, 0xb1, 0xf, 0xf, true);
+		const int apart = __popcll(lanes((curr & 1u) != 0u && beside != curr));
+		if (apart < kStageMin)
+			run(std::true_type{});
+		else
+			run(std::false_type{});
 	}
 }
 
