@@ -662,23 +662,65 @@ typedef __attribute__((address_space(3))) uint32_t LdsWord;
 typedef __attribute__((address_space(3))) char LdsByte;
 typedef __attribute__((address_space(3))) Pair LdsPair;
 typedef __attribute__((address_space(1))) char GlobalByte;
-// Stack rows in LDS, and how many of them move to private memory at once.
+// Stack rows in LDS, and how many of them move to device memory at once.
 // With the 4 KiB stage, 11 + 3 rows make 7,680 B per wave, six of the 1,280-B
 // units LDS is handed out in: 20 resident waves per CU, where 13 rows leave
 // 18 (primary rays 1,634 against 1,688 us, bounce rays 1,582 against 1,602 us
 // per 2.07 M on the 2.3 M-triangle terrain); 9 rows spill more and gain no
 // wave (1,659 / 1,607 us).
 constexpr int kRows = 11, kSpill = 5;
+
+// Where they move to: slots of kDeep entries per lane, one per wave that
+// needs any (rays deeper than 11 entries: 0.4 % of the bounce rays of a
+// 2.3 M-triangle terrain).  A wave claims a slot in the bitmap at its first
+// spill and gives it back when it ends.  LDS holds 21 of these waves per CU,
+// so 8,192 slots are never all taken by the waves of 256 CUs; a wave that
+// finds none counts a stack overflow.  Private memory would do, but a
+// queue's first launch with scratch allocates it for the whole machine (0.3
+// to 1.1 ms on each new stream).
+//
+// The entries are read and written at agent scope: a slot's next wave may
+// run on another XCD, whose L2 is not this one's.  A lane reads only what it
+// wrote itself, so nothing has to be acquired or released with the slot
+// beyond the wait for the last owner's stores; acquire and release would
+// invalidate and write back whole L2s (bounce rays 1,590 instead of 1,547
+// us).
+constexpr int kDeep = (kStack - kRows + kSpill - 1) / kSpill * kSpill;
+constexpr uint32_t kDeepSlots = 8192, kNoSlot = 0xffffffffu;
+__device__ uint32_t deep_slots[kDeepSlots / 32];
+__device__ uint32_t deep_entries[kDeepSlots * kDeep * kWave];
+
+// a free slot, or kNoSlot (the calling lane's search is bounded)
+__device__ inline uint32_t claim_deep_slot(uint32_t start) {
+	for (uint32_t i = 0; i < 2 * kDeepSlots / 32; ++i) {
+		const uint32_t w = (start + i) % (kDeepSlots / 32);
+		uint32_t used = __hip_atomic_load(&deep_slots[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		for (int tries = 0; tries < 32 && used != 0xffffffffu; ++tries) {
+			const uint32_t bit = (uint32_t)__ffs((int)~used) - 1u;
+			const uint32_t old = __hip_atomic_fetch_or(&deep_slots[w], 1u << bit, __ATOMIC_RELAXED,
+			                                           __HIP_MEMORY_SCOPE_AGENT);
+			if (!(old >> bit & 1u)) return w * 32u + bit;
+			used = old;
+		}
+	}
+	return kNoSlot;
+}
+
+__device__ inline void release_deep_slot(uint32_t slot) {
+	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the entries' stores
+	__hip_atomic_fetch_and(&deep_slots[slot / 32u], ~(1u << (slot % 32u)), __ATOMIC_RELAXED,
+	                       __HIP_MEMORY_SCOPE_AGENT);
+}
 // At least this many lanes whose neighbour stands at another inner node make
 // a wave take its next round of steps through the stage.  Of thresholds 12,
 // 24, 36 and never: primary rays 1,793 / 1,698 / 1,683 / 1,603 us, bounce
 // rays 1,617 / 1,613 / 1,609 / 2,141 us (16 rows, same scene).
 constexpr int kStageMin = 36;
 
-// The largest x with x < ct && x <= tmax, for ct > 0 (-inf for a NaN tmax,
-// which accepts nothing).
-__device__ inline float accept_limit(float ct, float tmax) {
-	const float below = __uint_as_float(__float_as_uint(ct) - 1u);
+// The largest x with x < FLT_MAX && x <= tmax (-inf for a NaN tmax, which
+// accepts nothing).
+__device__ inline float accept_limit(float tmax) {
+	const float below = __uint_as_float(__float_as_uint(FLT_MAX) - 1u);
 	return tmax == tmax ? fminf(below, tmax) : -__builtin_inff();
 }
 
@@ -707,15 +749,14 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 	// register (`top`), the ones below it in rows 1 .. kRows, the lowest of
 	// them the bottom mark kIdle; `sp` points at the last of those rows (row
 	// 0 while there is none).  Row 0 is read, and its value dropped, when a
-	// lane pops the mark (sp is row -1 from then on, and the idle lane may
-	// still read it); row kRows + 1 is written when a lane whose rows are
+	// lane pops the mark (sp is row -1 from then on; the idle lane may still
+	// read there, and write row 0); row kRows + 1 is written when a lane whose rows are
 	// full takes a step.  A push beyond kRows first moves the lowest kSpill
-	// rows (or what is left of STACK) to private memory, `deep`, of which
-	// `spilled` entries are in use.
+	// rows (or what is left of STACK) to the wave's deep slot, `spilled`
+	// entries of this lane.
 	__shared__ uint32_t stack[(kRows + 3) * BLOCK];
 	__shared__ float4 stage[BLOCK / kWave][4][kWave];   // see run
-	constexpr int kDeep = STACK - kRows;
-	uint32_t deep[kDeep + kSpill];
+	constexpr int kMaxSpilled = STACK - kRows;
 	int spilled = 0;
 	const int lt = threadIdx.x;
 	const int lane = __lane_id();
@@ -733,6 +774,9 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 	LdsWord *bottom = (LdsWord *)&stack[BLOCK + lt];
 	asm("" : "+v"(bottom));   // one register, not lane base + offset
 	LdsWord *const limit = bottom + kRows * BLOCK;
+	// the wave's deep slot, or kNoSlot, stands in row -1 of every lane, which
+	// nothing else writes
+	bottom[-BLOCK] = kNoSlot;
 	LdsWord *sp = bottom;
 	const int wave = __builtin_amdgcn_readfirstlane(lt / kWave);
 	const int quad = lane & 3;
@@ -742,14 +786,31 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 
 	uint32_t curr = kIdle, top = kIdle, ray = kNoRay;
 	bool exhausted = false;
+	// The wave's own run of rays [run_at, run_end), taken from the queue with
+	// one atomic: what it needs now or, if more, a share of what is left.
+	// The queue is one word whose atomics take turns (about 7 ns each), which
+	// bounded launches of short rays when every refill took one: 64 meshes'
+	// build and 4.45 M-ray trace 1,922 us, with shares of 1/4, 1/2 and 1/1 of
+	// an even split 1,688 / 1,584 / 1,613 us.  Long rays lose to uneven ends
+	// what larger shares save (primary rays of the 2.3 M-triangle terrain
+	// 1,621 us, then 1,623 / 1,661 / 1,963; bounce rays 1,568, then 1,551 /
+	// 1,539 / 1,694), so one mesh takes 1/4 and a batch 1/2.
+	uint32_t run_at = 0, run_end = 0, left = n;
+	const uint32_t split = (BATCHED ? 2u : 4u) * gridDim.x * (BLOCK / kWave);
+	const int share = 32 - __builtin_clz(split);
+	// BATCHED: the last refill's mesh and its rays
+	uint32_t mesh_at = 0, mesh_first = 0, mesh_rays = 0;
 	uint32_t node_base = 0, tri_base = 0;
 	float ox = 0, oy = 0, oz = 0, dx = 0, dy = 0, dz = 0, yx = 0, yy = 0, yz = 0, tmax = 0;
-	// lim: the largest entry distance or hit distance still accepted,
-	// min(tmax, the float below ct), so that `x <= lim` is the reference's
-	// x < closest.t && x <= max_t
-	float ct = FLT_MAX, cb = 0, cg = 0, lim = 0;
-	uint32_t cref = 0;
-	bool fast = true;
+	// lim: the largest entry distance or hit distance still accepted: max_t
+	// and the float below closest.t, so that `x <= lim` is the reference's
+	// x < closest.t && x <= max_t.  A hit accepted at t makes it the float
+	// below t, so it stands for the closest t too (cref: kNoRay before that).
+	float cb = 0, cg = 0, lim = 0;
+	uint32_t cref = kNoRay;
+	auto closest_t = [&]() {
+		return cref != kNoRay ? __uint_as_float(__float_as_uint(lim) + 1u) : FLT_MAX;
+	};
 	// Rounds (of at most `steps` wave-steps) since the last refill.  Every
 	// wave-step advances at least one lane and each lane holds at most one
 	// ray per refill, so with a valid tree (at most 2 * nodes < kMaxSteps
@@ -760,6 +821,8 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 	const uint64_t round_limit = 64ull * kMaxSteps / (uint64_t)steps + 2;
 	uint64_t slow_lanes = 0;   // lanes whose ray takes the IEEE box test
 	uint64_t deep_lanes = 0;   // lanes with spilled stack entries
+
+	auto deep_at = [&](int i) { return &deep_entries[(bottom[-BLOCK] * kDeep + i) * kWave + lane]; };
 
 	// The reference's decision at an inner node (kernels.cu:818-835) for the
 	// lanes there, without branches: both children kept -> enter the nearer,
@@ -774,7 +837,7 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 		uint64_t hr = lanes(dr <= fr) & lanes(dr <= lim) & lanes(fr >= 0.0f);
 		if (slow_lanes != 0ull) {
 			bool sl = false, sr = false;
-			if (!fast) {
+			if (in_mask(slow_lanes)) {
 				const float4 *p = pairs + 4 * ((size_t)node_base + (curr >> 1));
 				const float4 q0 = p[0], q1 = p[1], q2 = p[2];
 				sl = box_test(q0.x, q0.z, q1.x, q1.z, q2.x, q2.z, ox, oy, oz, dx, dy, dz, dl);
@@ -789,33 +852,44 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 		const uint32_t near_w = enter_left ? wl : wr, far_w = enter_left ? wr : wl;
 		curr = any ? near_w : top;
 		top = push ? far_w : (any ? top : below);
-		const uint64_t over = both & lanes(sp == limit);
-		if (over != 0ull) {
-			if (in_mask(over)) {
-				if (spilled < kDeep) {
-					const int m = min(kSpill, kDeep - spilled);
-#pragma nounroll
-					for (int i = 0; i < m; ++i) deep[spilled + i] = bottom[(1 + i) * BLOCK];
-#pragma nounroll
-					for (int i = 1; i <= kRows + 1 - m; ++i) bottom[i * BLOCK] = bottom[(i + m) * BLOCK];
-					sp -= m * BLOCK;
-					spilled += m;
-				} else {
-					// a push beyond STACK entries ends the ray with an error count
-					// (STACK = kStack) or on the overflow list (STACK < kStack)
-					curr = kIdle;
-					sp = bottom - BLOCK;
-					if (STACK < kStack) {
-						ovf[1 + atomicAdd(ovf, 1u)] = ray;   // traced again
-						ray = kNoRay;
-					} else {
-						atomicAdd(err, 1u);
-					}
-				}
-			}
-			deep_lanes |= lanes(spilled != 0);
-		}
 		sp += push ? BLOCK : (any ? 0 : -BLOCK);
+	};
+
+	// After an inner-node step, for the whole wave (its slot and deep_lanes are
+	// the wave's, so nothing here runs for some of its lanes only but what
+	// is under `full`): lanes that pushed beyond row kRows spill; beyond
+	// STACK entries the ray ends with an error count (STACK = kStack) or on
+	// the overflow list (STACK < kStack).
+	auto spill = [&]() {
+		const uint64_t over = lanes(sp == limit + BLOCK);
+		if (over == 0ull) return;
+		uint32_t slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)bottom[-BLOCK]);
+		if (slot == kNoSlot) {
+			if (lane == 0) slot = claim_deep_slot(blockIdx.x);
+			slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)slot);
+			bottom[-BLOCK] = slot;
+		}
+		const bool full = sp == limit + BLOCK;
+		if (full && spilled < kMaxSpilled && slot != kNoSlot) {
+			const int m = min(kSpill, kMaxSpilled - spilled);
+			for (int i = 0; i < kSpill; ++i)   // the slot has room for whole groups
+				__hip_atomic_store(deep_at(spilled + i), bottom[(1 + i) * BLOCK], __ATOMIC_RELAXED,
+				                   __HIP_MEMORY_SCOPE_AGENT);
+#pragma nounroll
+			for (int i = 1; i <= kRows + 1 - m; ++i) bottom[i * BLOCK] = bottom[(i + m) * BLOCK];
+			sp -= m * BLOCK;
+			spilled += m;
+		} else if (full) {
+			curr = kIdle;
+			sp = bottom - BLOCK;
+			if (STACK < kStack) {
+				ovf[1 + atomicAdd(ovf, 1u)] = ray;   // traced again
+				ray = kNoRay;
+			} else {
+				atomicAdd(err, 1u);
+			}
+		}
+		deep_lanes = lanes(spilled != 0);
 	};
 
 	// Up to `steps` wave-steps.  Each is an inner-node step or a leaf step
@@ -872,6 +946,7 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 						          yz, dr, fr);
 						decide(dl, fl, dr, fr, words.x, words.y, below);
 					}
+					spill();
 				} else {
 					const uint32_t below = sp[0];
 					sp[BLOCK] = top;
@@ -907,6 +982,7 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 						decide(dl, fl, dr, fr, __float_as_uint(words[0]), __float_as_uint(words[1]),
 						       below);
 					}
+					spill();
 				}
 			} else if (!(curr & 1u) && curr != kIdle) {
 				uint32_t i = curr >> 1;
@@ -924,8 +1000,8 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 					if (tri_test(v0.x, v0.y, v0.z, v1.x, v1.y, v1.z, v2.x, v2.y, v2.z, ox, oy, oz,
 					             dx, dy, dz, t, be, ga)) {
 						if (t <= lim) {
-							ct = t; cb = be; cg = ga; cref = i;
-							lim = accept_limit(t, tmax);
+							cb = be; cg = ga; cref = i;
+							lim = __uint_as_float(__float_as_uint(t) - 1u);
 							if (ANY_HIT) {
 								curr = kIdle;
 								break;
@@ -942,8 +1018,12 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 				if (spilled != 0 && sp == bottom && curr != kIdle) {
 					const int part = spilled % kSpill, m = part ? part : kSpill;
 					spilled -= m;
-#pragma nounroll
-					for (int i = 0; i < m; ++i) bottom[(1 + i) * BLOCK] = deep[spilled + i];
+					uint32_t back[kSpill];   // all on their way before the first is waited for
+					for (int i = 0; i < kSpill; ++i) 
+						back[i] = __hip_atomic_load(deep_at(spilled + i), __ATOMIC_RELAXED,
+						                            __HIP_MEMORY_SCOPE_AGENT);
+					for (int i = 0; i < kSpill; ++i)
+						if (i < m) bottom[(1 + i) * BLOCK] = back[i];
 					sp += m * BLOCK;
 				}
 				deep_lanes = lanes(spilled != 0);
@@ -952,9 +1032,8 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 				// the treelet phase ends: its closest t (a real hit, or
 				// FLT_MAX), widened by seed_bound's margin, bounds the
 				// traversal of the whole tree
-				tmax = fminf(tmax, seed_bound(ct));
-				ct = FLT_MAX;
-				lim = accept_limit(ct, tmax);
+				lim = accept_limit(fminf(tmax, seed_bound(closest_t())));
+				cref = kNoRay;
 				curr = root_word;
 				top = kIdle;
 				sp = bottom;
@@ -967,46 +1046,69 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 	while (true) {
 		const uint64_t idle = lanes(curr == kIdle);
 		const int nidle = __popcll(idle);
-		if (nidle == kWave || (!exhausted && nidle >= refill_min)) {
+		if (nidle == kWave || ((!exhausted || run_at < run_end) && nidle >= refill_min)) {
 			// write the finished rays' records (t = FLT_MAX alone on a miss)
 			if (curr == kIdle && ray != kNoRay) {
-				if (ct != FLT_MAX) {
+				if (cref != kNoRay) {
 					rta_hit hres;
-					hres.t = ct; hres.beta = cb; hres.gamma = cg; hres.ref = cref;
+					hres.t = closest_t(); hres.beta = cb; hres.gamma = cg; hres.ref = cref;
 					hits[ray] = hres;
 				} else {
 					hits[ray].t = FLT_MAX;
 				}
 				ray = kNoRay;
 			}
-			if (exhausted) break;   // and every lane is idle
+			if (exhausted && run_at == run_end) break;   // and every lane is idle
 			rounds = 0;
-			const int leader = __ffsll((unsigned long long)idle) - 1;
-			uint32_t base = 0;
-			if (lane == leader) base = atomicAdd(queue, (uint32_t)nidle);
-			// readlane, not a shuffle: the result is wave-uniform for the
-			// compiler too, and with it the loop's control flow
-			base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);
-			if (base + (uint32_t)nidle >= n) exhausted = true;
+			const uint32_t have = run_end - run_at;
+			uint32_t next = run_end, next_end = run_end;
+			if (have < (uint32_t)nidle && !exhausted) {
+				const uint32_t take = max(left >> share, (uint32_t)nidle - have);
+				const int leader = __ffsll((unsigned long long)idle) - 1;
+				if (lane == leader) next = atomicAdd(queue, take);
+				// readlane, not a shuffle: the result is wave-uniform for the
+				// compiler too, and with it the loop's control flow
+				next = (uint32_t)__builtin_amdgcn_readlane((int)next, leader);
+				exhausted = next >= n || take >= n - next;
+				next = min(next, n);
+				next_end = exhausted ? n : next + take;
+				left = n - next_end;
+			}
+			const uint32_t rank = (uint32_t)__popcll(idle & lower);
+			const uint32_t my = rank < have ? run_at + rank : next + (rank - have);
+			const uint32_t my_end = rank < have ? run_end : next_end;
+			if (have < (uint32_t)nidle) {
+				run_at = min(next + ((uint32_t)nidle - have), next_end);
+				run_end = next_end;
+			} else {
+				run_at += (uint32_t)nidle;
+			}
+			int mesh = -1;   // BATCHED: a refilled lane's mesh
+			bool fast = true;
+			const uint64_t kept_slow = slow_lanes & ~idle;
 			if (curr == kIdle) {
-				const uint32_t my = base + (uint32_t)__popcll(idle & lower);
-				if (my < n) {
+				if (my < my_end) {
 					ray = ray_list ? ray_list[1 + my] : my;
 					ox = ro[3 * (size_t)ray + 0]; oy = ro[3 * (size_t)ray + 1]; oz = ro[3 * (size_t)ray + 2];
 					dx = rd[3 * (size_t)ray + 0]; dy = rd[3 * (size_t)ray + 1]; dz = rd[3 * (size_t)ray + 2];
 					tmax = rmax[ray];
 					if (BATCHED) {
-						// last mesh whose first ray is <= ray
-						int lo = 0, hi = n_meshes;
-						while (hi - lo > 1) {
-							const int mid = (lo + hi) >> 1;
-							if (meshes[mid].ray_off <= ray) lo = mid;
-							else hi = mid;
+						// last mesh whose first ray is <= ray: most often the last
+						// refill's
+						mesh = (int)mesh_at;
+						if (ray - mesh_first >= mesh_rays) {
+							int lo = 0, hi = n_meshes;
+							while (hi - lo > 1) {
+								const int mid = (lo + hi) >> 1;
+								if (meshes[mid].ray_off <= ray) lo = mid;
+								else hi = mid;
+							}
+							mesh = lo;
 						}
-						node_base = meshes[lo].node_off;
-						tri_base = meshes[lo].tri_off;
-						curr = root_words[lo];
-						fast = (flags[lo] & 1u) == 0u && ray_nz_ok(ox, oy, oz, dx, dy, dz);
+						node_base = meshes[mesh].node_off;
+						tri_base = meshes[mesh].tri_off;
+						curr = root_words[mesh];
+						fast = (flags[mesh] & 1u) == 0u && ray_nz_ok(ox, oy, oz, dx, dy, dz);
 					} else {
 						curr = root_word;
 						fast = scene_fast && ray_nz_ok(ox, oy, oz, dx, dy, dz);
@@ -1026,14 +1128,22 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 						}
 					}
 					yx = 1.0f / dx; yy = 1.0f / dy; yz = 1.0f / dz;
-					ct = FLT_MAX;
-					lim = accept_limit(ct, tmax);
+					lim = accept_limit(tmax);
+					cref = kNoRay;
 					top = kIdle;
 					sp = bottom;
 					spilled = 0;
 				}
 			}
-			slow_lanes = lanes(curr != kIdle && !fast);
+			if (BATCHED) {
+				const uint64_t took = lanes(mesh >= 0);
+				if (took != 0ull) {
+					mesh_at = (uint32_t)__builtin_amdgcn_readlane(mesh, 63 - __clzll((long long)took));
+					mesh_first = meshes[mesh_at].ray_off;
+					mesh_rays = meshes[mesh_at].n_rays;
+				}
+			}
+			slow_lanes = kept_slow | lanes(!fast);
 			deep_lanes = lanes(spilled != 0);
 			if (lanes(curr != kIdle) == 0ull) break;   // the queue was empty
 		}
@@ -1053,6 +1163,7 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 		else
 			run(std::false_type{});
 	}
+	if (lane == 0 && bottom[-BLOCK] != kNoSlot) release_deep_slot(bottom[-BLOCK]);
 }
 
 // ------------------------------------------------------- bouncing
