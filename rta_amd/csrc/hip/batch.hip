@@ -87,26 +87,22 @@ __global__ __launch_bounds__(kChunk) void batch_chunk_kernel(
 	                status, (int)m.n, (int)it.block, mesh_pack(m, it.mesh, pairs, tri4, flags));
 }
 
-// Merge level `level` (>= 1): level-`level` groups of a mesh cover
-// kChunk * kMergeFan^level leaves.
+// A merge level of every mesh that still has several groups.
 __global__ __launch_bounds__(kMergeThreads) void batch_merge_kernel(
     const BatchItem *__restrict__ items, const BatchMesh *__restrict__ meshes,
     rta_node *__restrict__ nodes, uint2 *__restrict__ ranges,
     const uint4 *__restrict__ in_slots, const uint32_t *__restrict__ in_counts,
     uint4 *__restrict__ out_slots, uint32_t *__restrict__ out_counts,
-    uint32_t *__restrict__ status, long long width, rta_node_pair *pairs, float4 *tri4,
-    uint32_t *flags) {
+    uint32_t *__restrict__ status, rta_node_pair *pairs, float4 *tri4, uint32_t *flags) {
 	const BatchItem it = items[blockIdx.x];
 	const BatchMesh m = meshes[it.mesh];
 	const uint32_t g0 = it.block * kMergeFan;
 	const int ng = (int)min((uint32_t)kMergeFan, it.groups - g0);
-	const uint32_t lo = (uint32_t)(it.block * width);
-	const uint32_t hi = (uint32_t)min((long long)m.n, (long long)(it.block + 1) * width);
 	const bool last = it.blocks == 1;
 	bottom_up_merge(nodes + m.node_off, ranges + m.tri_off,
 	                in_slots + (size_t)(m.chunk_off + g0) * kSlots, in_counts + m.chunk_off + g0, ng,
 	                last ? nullptr : out_slots + (size_t)(m.chunk_off + it.block) * kSlots,
-	                last ? nullptr : out_counts + m.chunk_off + it.block, status, lo, hi,
+	                last ? nullptr : out_counts + m.chunk_off + it.block, status,
 	                (int)m.n, mesh_pack(m, it.mesh, pairs, tri4, flags));
 }
 
@@ -374,14 +370,12 @@ static int batch_build(const char *name, rta_batch b, rta_triangle *tris, rta_no
 	                   items + p.chunk_items_off, p.d_meshes, nodes, w.boxes, w.codes, indices,
 	                   w.ranges, w.slots[0], w.counts[0], bu_status, pairs, tri4, flags);
 	RTA_LAUNCH_CHECK("batch_chunk_kernel");
-	long long width = kChunk;
 	for (size_t L = 0; L < p.merge_off.size(); ++L) {
-		width *= kMergeFan;
 		const int in = (int)(L & 1), outb = 1 - in;
 		hipLaunchKernelGGL(batch_merge_kernel, dim3((unsigned)p.merge_len[L]), dim3(kMergeThreads), 0,
 		                   st, items + p.merge_off[L], p.d_meshes, nodes,
 		                   w.ranges, w.slots[in], w.counts[in], w.slots[outb], w.counts[outb],
-		                   bu_status, width, pairs, tri4, flags);
+		                   bu_status, pairs, tri4, flags);
 		RTA_LAUNCH_CHECK("batch_merge_kernel");
 	}
 	if (pairs) {

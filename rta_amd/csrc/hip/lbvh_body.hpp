@@ -15,7 +15,6 @@ constexpr int kBoundsBlock = 1024;
 constexpr int kChunk = 1024;
 constexpr int kSlots = 128;
 constexpr int kMergeFan = 16;
-constexpr uint32_t kStateInner = 0xffffffffu; // leaf count of an inner node in the climb
 
 // ---------------------------------------------------------- wave helpers
 
@@ -160,20 +159,23 @@ __device__ inline void voxel_bounds_block(rta_aabb *__restrict__ bounds,
 
 // ------------------------------------------------ stage 3: Morton codes
 
-// The code of triangle i of a mesh.  d = GRIDSIZE/(max-min) is formed per
-// thread with the same correctly rounded division the reference does once on
-// the host (lbvh-kernels.cu:414-417), so every thread sees the identical d.
-__device__ inline uint32_t morton_of(const rta_float3 *__restrict__ centers,
-                                     const rta_aabb *__restrict__ bounds, int i) {
-	const rta_aabb vb = *bounds;
+// The code of a centroid.  d = GRIDSIZE/(max-min) is formed per thread with
+// the same correctly rounded division the reference does once on the host
+// (lbvh-kernels.cu:414-417), so every thread sees the identical d.
+__device__ inline uint32_t morton_code(const rta_float3 &c, const rta_aabb &vb) {
 	const float dx = 1024.0f / (vb.max.x - vb.min.x);
 	const float dy = 1024.0f / (vb.max.y - vb.min.y);
 	const float dz = 1024.0f / (vb.max.z - vb.min.z);
-	const rta_float3 c = centers[i];
 	const uint32_t x = f2u_rz_sat((c.x - vb.min.x) * dx);
 	const uint32_t y = f2u_rz_sat((c.y - vb.min.y) * dy);
 	const uint32_t z = f2u_rz_sat((c.z - vb.min.z) * dz);
 	return morton_encode_10bit(x, y, z);
+}
+
+// the code of triangle i of a mesh
+__device__ inline uint32_t morton_of(const rta_float3 *__restrict__ centers,
+                                     const rta_aabb *__restrict__ bounds, int i) {
+	return morton_code(centers[i], *bounds);
 }
 
 // ----------------------------------------- stage 5: Karras hierarchy
@@ -304,7 +306,9 @@ __device__ inline void karras_node(rta_node *__restrict__ nodes, uint32_t *__res
 //           keyed by split), until one block covers all leaves and reaches
 //           the root.
 // No step needs device-scope cache maintenance; results do not depend on
-// the schedule.
+// the schedule.  A merge level of the 2.3 M-triangle terrain takes 18 us (35
+// with a split table and scalar records), of an 82 k-triangle sphere 13 (25),
+// of a 5 k-triangle one 10 (18).
 
 __device__ inline rta_aabb union_lr(const rta_aabb &lb, const rta_aabb &rb) {
 	rta_aabb u;
@@ -369,29 +373,6 @@ __device__ inline int delta_at(const uint32_t *__restrict__ codes, long long i, 
 	return __clz((int)(a ^ b));
 }
 
-// A completed node during the climb.
-struct ClimbNode {
-	uint32_t l, r;     // sorted range
-	int dl, dr;        // delta(l - 1), delta(r)
-	rta_aabb box;
-	uint32_t elems;    // kStateInner for an inner node, else the leaf's triangle count
-	uint32_t tris;     // the leaf's first triangle
-};
-
-// its parent's split, and its own index there (r as a left child, l as a
-// right child); the root (dl = dr = -1) has neither
-__device__ inline bool is_left_child(const ClimbNode &c) { return c.dr > c.dl; }
-__device__ inline uint32_t node_index(const ClimbNode &c, uint32_t leaf0) {
-	if (c.l == c.r) return leaf0 + c.l;
-	return is_left_child(c) ? c.r : c.l;
-}
-
-// a frontier entry: index, range, deltas (+1, a byte each)
-__device__ inline uint4 frontier_entry(const ClimbNode &c, uint32_t leaf0) {
-	return make_uint4(node_index(c, leaf0), c.l, c.r,
-	                  (uint32_t)(c.dl + 1) | ((uint32_t)(c.dr + 1) << 8));
-}
-
 // the whole node: link words and box, as two 16-byte stores
 __device__ inline void store_node(rta_node *node, uint2 links, const rta_aabb &b) {
 	uint4 *o = reinterpret_cast<uint4 *>(node);
@@ -400,48 +381,183 @@ __device__ inline void store_node(rta_node *node, uint2 links, const rta_aabb &b
 	                  __float_as_uint(b.max.z));
 }
 
-// leaf state of a finished node from its link words
-__device__ inline void node_state(uint2 links, uint32_t &elems, uint32_t &tris) {
-	elems = link_inner(links.x) ? kStateInner : links.x >> 1;
-	tris = links.y;
+// Bottom-up over E consecutive items of a mesh in one workgroup: the leaves
+// of a chunk (level 1) or the frontier entries of some groups (above).  Item
+// i covers the sorted positions [pos(i), pos(i + 1)); the items are adjacent
+// and in order, so a node is a run of items [a, b] and a split is the
+// boundary j between items j and j + 1.
+//
+// The climbs touch LDS only.  Every child arriving at a boundary writes its
+// record (box, far item, delta there, leaf state: two 16-byte words) under
+// that boundary and its side, then counts its arrival; the second arrival
+// reads its sibling's record and climbs on with the parent.  Fences are
+// LDS-only.  Afterwards each boundary whose two children arrived writes the
+// parent's whole node, range and pair record from the two records, one
+// boundary per thread; a node whose parent stays incomplete (its sibling
+// reaches beyond the items) joins the frontier, which is written in order.
+//
+// A leaf holds the triangles of its range: a merge of leaves [l, s] and
+// [s + 1, r] gives tris = l and elems = r - l + 1, so its state is one bit.
+//
+// What bounds it: the chain of dependent LDS round trips of the climbs and
+// the instructions of waves with few lanes still climbing.
+struct ClimbRecord {
+	float4 lo;   // min.x, min.y, min.z, max.x
+	float4 hi;   // max.y, max.z, far item, delta + 1 at the far end | inner << 8
+};
+constexpr uint32_t kArriveRight = 0x10000u;   // visit count of a right child (a left one adds 1)
+constexpr uint32_t kNoFront = 0xffffffffu, kFrontInner = 0x80000000u;   // frontier marks
+constexpr uint32_t kEntryInner = 0x10000u;    // frontier entry: an inner node
+constexpr uint32_t kInnerBit = 0x100u;
+
+template <int E>
+struct ClimbShared {
+	ClimbRecord rec[2][E];       // per side (0: the left child) and boundary
+	uint32_t visit[E];           // arrivals per boundary; then the frontier
+	int8_t delta[E + 4];         // delta at the start of item i; [items]: at the end
+	uint32_t wave_count[16];
+};
+
+// One item, before the climb.
+struct ClimbItem {
+	rta_aabb box;
+	bool inner;
+};
+
+// The climb of item i.
+template <int E>
+__device__ inline void climb(ClimbShared<E> &sh, int i, int items, const ClimbItem &it) {
+	rta_aabb box = it.box;
+	bool inner = it.inner;
+	int a = i, b = i;
+	int dl = sh.delta[i], dr = sh.delta[i + 1];
+	for (int level = 0; level < 128; ++level) {
+		if (dl < 0 && dr < 0) break;      // the root of the mesh
+		const bool left = dr > dl;        // the left child of boundary b, else the right of a - 1
+		// the sibling lies beyond the items: an edge record (boundary items - 1
+		// is never formed here, its slots take the last and the first node)
+		const bool edge = left ? b + 1 == items : a == 0;
+		const int j = edge ? items - 1 : (left ? b : a - 1);
+		ClimbRecord &mine = sh.rec[left ? 0 : 1][j];
+		mine.lo = make_float4(box.min.x, box.min.y, box.min.z, box.max.x);
+		mine.hi = make_float4(box.max.y, box.max.z, __uint_as_float((uint32_t)(left ? a : b)),
+		                      __uint_as_float((uint32_t)((left ? dl : dr) + 1) |
+		                                      (inner ? kInnerBit : 0u)));
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+		const uint32_t old = atomicAdd(&sh.visit[j], left ? 1u : kArriveRight);
+		if (edge || old == 0u) break;     // else the sibling forms the parent
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+		const ClimbRecord sib = sh.rec[left ? 1 : 0][j];
+		const rta_aabb sbox = {{sib.lo.x, sib.lo.y, sib.lo.z}, {sib.lo.w, sib.hi.x, sib.hi.y}};
+		const int far = (int)__float_as_uint(sib.hi.z);
+		const uint32_t meta = __float_as_uint(sib.hi.w);
+		const int dfar = (int)(meta & 0xffu) - 1, ds = left ? dr : dl;
+		// both leaves and equal codes at the boundary: one leaf
+		inner = inner || (meta & kInnerBit) != 0u || ds < 32;
+		box = left ? union_lr(box, sbox) : union_lr(sbox, box);
+		if (left) { b = far; dr = dfar; }
+		else { a = far; dl = dfar; }
+	}
 }
 
-// The parent of lc = [l, s] and rc = [s+1, r]: its whole node, range and,
-// after a merge, the cleared leaf-end mark; returns it, its index in x.
-__device__ inline ClimbNode form_parent(const ClimbNode &lc, const ClimbNode &rc, uint32_t s,
-                                        uint32_t leaf0, rta_node *__restrict__ nodes,
-                                        uint2 *__restrict__ ranges, const PackOut &pk,
-                                        uint32_t &x) {
-	ClimbNode p;
-	p.l = lc.l;
-	p.r = rc.r;
-	p.dl = lc.dl;
-	p.dr = rc.dr;
-	p.box = union_lr(lc.box, rc.box);
-	const uint32_t lid = lc.l == lc.r ? leaf0 + s : s;
-	const uint32_t rid = rc.l == rc.r ? leaf0 + s + 1u : s + 1u;
-	const bool merge = lc.dr >= 32 && lc.elems != kStateInner && rc.elems != kStateInner;
-	p.elems = merge ? lc.elems + rc.elems : kStateInner;
-	p.tris = merge ? (lc.tris < rc.tris ? lc.tris : rc.tris) : 0u;
-	x = node_index(p, leaf0);
-	store_node(&nodes[x], merge ? make_uint2(p.elems << 1, p.tris) : make_uint2((lid << 1) | 1u, rid),
-	           p.box);
-	ranges[x] = make_uint2(p.l, p.r);
-	if (merge && pk.tri4) clear_leaf_end(pk.tri4, s);
-	return p;
+// After the climbs of all items and a barrier: thread t takes boundaries (and
+// frontier items) t, t + threads, ...  All threads of the block call it.
+// Returns the frontier's size.
+template <int E, int THREADS, class Pos>
+__device__ inline uint32_t emit_nodes(ClimbShared<E> &sh, int items, const Pos &pos,
+                                      rta_node *__restrict__ nodes, uint2 *__restrict__ ranges,
+                                      uint4 *__restrict__ slots, int n, const PackOut &pk) {
+	const int t = threadIdx.x;
+	const uint32_t leaf0 = (uint32_t)(n - 1);
+	constexpr int kPer = E / THREADS;
+	static_assert(E % THREADS == 0 && THREADS % kWave == 0 && THREADS <= 16 * kWave, "whole rounds");
+	bool slow = false;
+	uint32_t v[kPer];
+#pragma unroll
+	for (int k = 0; k < kPer; ++k) {
+		const int j = t + k * THREADS;
+		v[k] = j < items ? sh.visit[j] : 0u;
+		if (j + 1 >= items || v[k] != 1u + kArriveRight) continue;
+		const ClimbRecord L = sh.rec[0][j], R = sh.rec[1][j];
+		const int a = (int)__float_as_uint(L.hi.z), b = (int)__float_as_uint(R.hi.z);
+		const uint32_t lm = __float_as_uint(L.hi.w), rm = __float_as_uint(R.hi.w);
+		const uint32_t l = pos(a), s = pos(j + 1) - 1u, r = pos(b + 1) - 1u;
+		const int dl = (int)(lm & 0xffu), dr = (int)(rm & 0xffu), ds = sh.delta[j + 1];
+		const rta_aabb lb = {{L.lo.x, L.lo.y, L.lo.z}, {L.lo.w, L.hi.x, L.hi.y}};
+		const rta_aabb rb = {{R.lo.x, R.lo.y, R.lo.z}, {R.lo.w, R.hi.x, R.hi.y}};
+		const bool linner = (lm & kInnerBit) != 0u, rinner = (rm & kInnerBit) != 0u;
+		const bool merge = ds >= 32 && !linner && !rinner;
+		// the node's index: r as a left child, l as a right child or the root
+		const uint32_t x = dr > dl ? r : l;
+		const uint32_t lid = l == s ? leaf0 + s : s, rid = r == s + 1u ? leaf0 + r : s + 1u;
+		store_node(&nodes[x], merge ? make_uint2((r - l + 1u) << 1, l) : make_uint2((lid << 1) | 1u, rid),
+		           union_lr(lb, rb));
+		ranges[x] = make_uint2(l, r);
+		if (merge) {
+			if (pk.tri4) clear_leaf_end(pk.tri4, s);
+		} else if (pk.pairs) {
+			const uint32_t lw = linner ? (s << 1) | 1u : l << 1;
+			const uint32_t rw = rinner ? ((s + 1u) << 1) | 1u : (s + 1u) << 1;
+			if (!write_pair(pk.pairs, x, lb, rb, lw, rw, lid, rid)) slow = true;
+		}
+	}
+	if (pk.flags && __syncthreads_or(slow) && t == 0) atomicOr(pk.flags, 1u);
+	__syncthreads();
+	// The frontier, by first item: nodes that are the only arrival at their
+	// boundary, and the edge records.
+#pragma unroll
+	for (int k = 0; k < kPer; ++k) sh.visit[t + k * THREADS] = kNoFront;
+	__syncthreads();
+#pragma unroll
+	for (int k = 0; k < kPer; ++k) {
+		const int j = t + k * THREADS;
+		const bool edge = j + 1 == items;
+		if (v[k] == 0u || (!edge && v[k] == 1u + kArriveRight)) continue;
+		if (v[k] & 1u) {
+			const float4 hi = sh.rec[0][j].hi;
+			sh.visit[__float_as_uint(hi.z)] =
+			    (uint32_t)j | (__float_as_uint(hi.w) & kInnerBit ? kFrontInner : 0u);
+		}
+		if (v[k] & kArriveRight) {
+			const float4 hi = sh.rec[1][j].hi;
+			sh.visit[edge ? 0 : j + 1] =
+			    __float_as_uint(hi.z) | (__float_as_uint(hi.w) & kInnerBit ? kFrontInner : 0u);
+		}
+	}
+	__syncthreads();
+	uint32_t total = 0;
+#pragma unroll
+	for (int k = 0; k < kPer; ++k) {
+		const int a = t + k * THREADS;
+		const uint32_t f = a < items ? sh.visit[a] : kNoFront;
+		const uint64_t has = __ballot(f != kNoFront);
+		const int wave = t / kWave;
+		if (__lane_id() == 0) sh.wave_count[wave] = (uint32_t)__popcll(has);
+		__syncthreads();
+		uint32_t before = total, all = 0;
+		for (int w = 0; w < THREADS / kWave; ++w) {
+			const uint32_t c = sh.wave_count[w];
+			before += w < wave ? c : 0u;
+			all += c;
+		}
+		__syncthreads();
+		total += all;
+		if (f == kNoFront) continue;
+		const uint32_t rank = before + (uint32_t)__popcll(has & ((1ull << __lane_id()) - 1ull));
+		const int b = (int)(f & ~kFrontInner);
+		const uint32_t l = pos(a), r = pos(b + 1) - 1u;
+		const int dl = sh.delta[a], dr = sh.delta[b + 1];
+		const uint32_t x = l == r ? leaf0 + l : (dr > dl ? r : l);
+		if (slots && rank < (uint32_t)kSlots)
+			slots[rank] = make_uint4(x, l, r, (uint32_t)(dl + 1) | ((uint32_t)(dr + 1) << 8) |
+			                                      (f & kFrontInner ? kEntryInner : 0u));
+	}
+	return total;
 }
 
 // Level 1 for leaves [chunk*kChunk, +kChunk) of a mesh: every leaf's node,
 // every node completed inside the chunk, and the frontier in slots[0..kSlots)
-// with its size in *count.  The climbs touch LDS only: every child arriving
-// at a split of the chunk writes its record (box, far end, the delta there,
-// leaf state) under that split and its side, then counts its arrival; the
-// second arrival reads its sibling's record and climbs on with the parent.
-// Afterwards each split whose two children arrived writes the parent's
-// node, range and pair record from the two records, one split per thread,
-// and a split with one arrival gives a frontier entry.
-constexpr uint16_t kInner16 = 0xffffu;      // record: an inner node
-constexpr uint32_t kArriveRight = 0x10000u; // visit count of a right child (a left one adds 1)
+// with its size in *count.
 __device__ inline void bottom_up_chunk(rta_node *__restrict__ nodes,
                                        const rta_aabb *__restrict__ boxes,
                                        const uint32_t *__restrict__ codes,
@@ -450,304 +566,93 @@ __device__ inline void bottom_up_chunk(rta_node *__restrict__ nodes,
                                        uint4 *__restrict__ slots, uint32_t *__restrict__ count,
                                        uint32_t *__restrict__ status, int n, int chunk,
                                        PackOut pk = PackOut{}) {
-	// records per split base + j and side (0: the left child, 1: the right)
-	__shared__ float rbox[2][6][kChunk];
-	__shared__ uint16_t rfar[2][kChunk];     // the far end of the child's range, - base
-	__shared__ uint16_t relems[2][kChunk];   // a leaf's triangle count, or kInner16
-	__shared__ uint16_t rtris[2][kChunk];    // a leaf's first position, - base
-	__shared__ int8_t rdfar[2][kChunk];      // delta at the far end
-	__shared__ uint32_t lvisit[kChunk];      // arrivals per split
-	__shared__ int8_t ldelta[kChunk + 1];    // delta(base + j - 1)
-	__shared__ uint4 front[kSlots];
-	__shared__ uint32_t nfront;
-
+	__shared__ ClimbShared<kChunk> sh;
 	const int t = threadIdx.x;
 	const uint32_t base = (uint32_t)chunk * kChunk;
-	const uint32_t leaf0 = (uint32_t)(n - 1);
-	const uint32_t end = min(base + (uint32_t)kChunk, (uint32_t)n);
-	const uint32_t cnt = end - base;
-	const uint32_t k = base + t;
-	lvisit[t] = 0;
-	if (t == 0) nfront = 0;
-	if ((uint32_t)t <= cnt) ldelta[t] = (int8_t)delta_at(codes, (long long)base + t - 1, n);
-	if (t == 0 && cnt == (uint32_t)kChunk) ldelta[kChunk] = (int8_t)delta_at(codes, (long long)end - 1, n);
-	const bool live = k < (uint32_t)n;
-	ClimbNode c;
-	if (live) {
-		c.l = c.r = k;
-		c.box = boxes[indices[k]];
-		c.elems = 1u;
-		c.tris = k;
-		store_node(&nodes[leaf0 + k], make_uint2(1u << 1, k), c.box);
+	const int items = (int)min((uint32_t)kChunk, (uint32_t)n - base);
+	ClimbItem it{{}, false};
+	if (t < items) {
+		const uint32_t k = base + t;
+		it.box = boxes[indices[k]];
+		store_node(&nodes[(uint32_t)(n - 1) + k], make_uint2(1u << 1, k), it.box);
 	}
-	auto push = [&](const uint4 &e) {
-		const uint32_t slot = atomicAdd(&nfront, 1u);
-		if (slot < (uint32_t)kSlots) front[slot] = e;
-		else atomicOr(status, (uint32_t)RTA_LBVH_FRONTIER_OVERFLOW);
-	};
-	// the child that arrived at split base + j on `side`
-	auto record = [&](uint32_t j, int side) -> ClimbNode {
-		ClimbNode a;
-		a.box.min = {rbox[side][0][j], rbox[side][1][j], rbox[side][2][j]};
-		a.box.max = {rbox[side][3][j], rbox[side][4][j], rbox[side][5][j]};
-		const uint32_t far = base + rfar[side][j];
-		const int dfar = rdfar[side][j], ds = ldelta[j + 1];
-		if (side == 0) { a.l = far; a.r = base + j; a.dl = dfar; a.dr = ds; }
-		else { a.l = base + j + 1u; a.r = far; a.dl = ds; a.dr = dfar; }
-		const uint16_t e = relems[side][j];
-		a.elems = e == kInner16 ? kStateInner : (uint32_t)e;
-		a.tris = base + rtris[side][j];
-		return a;
-	};
+	sh.visit[t] = 0;
+	for (int i = t; i <= items; i += kChunk)
+		sh.delta[i] = (int8_t)delta_at(codes, (long long)base + i - 1, n);
 	__syncthreads();
-
-	if (live) {
-		c.dl = ldelta[t];
-		c.dr = ldelta[t + 1];
-		for (int level = 0; level < 128; ++level) {
-			if (c.dl < 0 && c.dr < 0) break;   // the root of the mesh
-			const bool left = is_left_child(c);
-			const uint32_t s = left ? c.r : c.l - 1u;
-			if (s < base || s + 1u >= end) {
-				push(frontier_entry(c, leaf0));   // the sibling starts in another chunk
-				break;
-			}
-			const uint32_t j = s - base;
-			const int side = left ? 0 : 1;
-			rbox[side][0][j] = c.box.min.x; rbox[side][1][j] = c.box.min.y; rbox[side][2][j] = c.box.min.z;
-			rbox[side][3][j] = c.box.max.x; rbox[side][4][j] = c.box.max.y; rbox[side][5][j] = c.box.max.z;
-			rfar[side][j] = (uint16_t)((left ? c.l : c.r) - base);
-			rdfar[side][j] = (int8_t)(left ? c.dl : c.dr);
-			const bool inner = c.elems == kStateInner;
-			relems[side][j] = inner ? kInner16 : (uint16_t)c.elems;
-			rtris[side][j] = inner ? (uint16_t)0 : (uint16_t)(c.tris - base);
-			__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-			const uint32_t old = atomicAdd(&lvisit[j], left ? 1u : kArriveRight);
-			if (old == 0u) break;
-			__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-			const ClimbNode sib = record(j, left ? 1 : 0);
-			const ClimbNode &lc = left ? c : sib;
-			const ClimbNode &rc = left ? sib : c;
-			ClimbNode p;
-			p.l = lc.l; p.r = rc.r; p.dl = lc.dl; p.dr = rc.dr;
-			p.box = union_lr(lc.box, rc.box);
-			const bool merge = lc.dr >= 32 && lc.elems != kStateInner && rc.elems != kStateInner;
-			p.elems = merge ? lc.elems + rc.elems : kStateInner;
-			p.tris = merge ? (lc.tris < rc.tris ? lc.tris : rc.tris) : 0u;
-			c = p;
-		}
+	if (t < items) climb(sh, t, items, it);
+	__syncthreads();
+	const uint32_t total = emit_nodes<kChunk, kChunk>(
+	    sh, items, [&](int i) { return base + (uint32_t)i; }, nodes, ranges, slots, n, pk);
+	if (t == 0) {
+		if (total > (uint32_t)kSlots) atomicOr(status, (uint32_t)RTA_LBVH_FRONTIER_OVERFLOW);
+		*count = min(total, (uint32_t)kSlots);
 	}
-	__syncthreads();
-
-	// write-out, per split s = base + t of the chunk: the parent when both
-	// children arrived, a frontier entry when one did (its sibling reaches
-	// beyond the chunk)
-	bool slow = false;
-	if ((uint32_t)t + 1u < cnt) {
-		const uint32_t v = lvisit[t];
-		if (v == 1u + kArriveRight) {
-			const ClimbNode lc = record(t, 0), rc = record(t, 1);
-			const uint32_t s = base + t;
-			uint32_t x;
-			form_parent(lc, rc, s, leaf0, nodes, ranges, pk, x);
-			const bool merged = lc.dr >= 32 && lc.elems != kStateInner && rc.elems != kStateInner;
-			if (!merged && pk.pairs) {
-				const uint32_t lid = lc.l == lc.r ? leaf0 + s : s;
-				const uint32_t rid = rc.l == rc.r ? leaf0 + s + 1u : s + 1u;
-				const uint32_t lw = lc.elems == kStateInner ? (s << 1) | 1u : lc.tris << 1;
-				const uint32_t rw = rc.elems == kStateInner ? ((s + 1u) << 1) | 1u : rc.tris << 1;
-				slow = !write_pair(pk.pairs, x, lc.box, rc.box, lw, rw, lid, rid);
-			}
-		} else if (v != 0u) {
-			push(frontier_entry(record(t, v == 1u ? 0 : 1), leaf0));
-		}
-	}
-	if (pk.flags && __syncthreads_or(slow) && t == 0) atomicOr(pk.flags, 1u);
-	__syncthreads();
-	const uint32_t nf = min(nfront, (uint32_t)kSlots);
-	if ((uint32_t)t < nf) slots[t] = front[t];
-	if (t == 0) *count = nf;
 }
 
 // Level k >= 2 for one mesh: merges the frontier slots of the ng chunks of
 // the previous level starting at in_slots/in_counts (kSlots entries per
-// chunk, at most kMergeEntries in all), whose leaves span [lo, hi); the new
-// frontier goes to out_slots / *out_count when given.  Thread t climbs from
-// entries t, t + kMergeThreads, ... in turn (a climb never waits, so one
-// thread may hold both children of a split).  The climbs touch LDS only:
-// every arrival at a split writes its record (far end, the deltas there and
-// at the split, box, leaf state) into its entry's record slot and then
-// claims the split's entry of an open-addressing table with one 64-bit
-// compare-and-swap of (split, record + 1); a climb that finds the split
-// already there is the second and forms the parent from the first's
-// record.  Only the first arrival stops, so a record is read only after its
-// last write.  A block sees at most kMergeEntries distinct splits, so the
-// table (half full at most) never runs out.  A child whose sibling lies
-// beyond [lo, hi) -- its parent's split is outside, or its entry holds a
-// single arrival at the end -- joins the new frontier.
+// chunk, in order); the new frontier goes to out_slots / *out_count when
+// given (the last level has none).
 constexpr int kMergeThreads = 1024;
 constexpr int kMergeEntries = kMergeFan * kSlots;
-constexpr int kTableBits = 12;
-constexpr int kTable = 1 << kTableBits;              // >= 2 kMergeEntries
-constexpr uint64_t kEmpty = ~0ull;                   // free table entry
-// record word once both children arrived: kFormed, or kFormedInner | x for
-// an inner parent x that needs its pair record
-constexpr uint32_t kFormed = 0xffffffffu;
-constexpr uint32_t kFormedInner = 0x80000000u;
-static_assert(kTable >= 2 * kMergeEntries, "merge table at most half full");
 __device__ inline void bottom_up_merge(rta_node *__restrict__ nodes, uint2 *__restrict__ ranges,
                                        const uint4 *__restrict__ in_slots,
                                        const uint32_t *__restrict__ in_counts, int ng,
                                        uint4 *__restrict__ out_slots,
                                        uint32_t *__restrict__ out_count,
-                                       uint32_t *__restrict__ status, uint32_t lo, uint32_t hi,
-                                       int n, PackOut pk = PackOut{}) {
-	__shared__ uint32_t gcount[kMergeFan];
-	// kEmpty, or (split << 32) | (the first arrival's record + 1, or the
-	// formed mark)
-	__shared__ uint64_t table[kTable];
-	// records, one per entry
-	__shared__ float rbox[6][kMergeEntries];
-	__shared__ uint32_t rfar[kMergeEntries];     // far end of the child's range
-	__shared__ uint32_t relems[kMergeEntries];
-	__shared__ uint32_t rtris[kMergeEntries];
-	__shared__ int8_t rdfar[kMergeEntries];      // delta at the far end
-	__shared__ int8_t rdnear[kMergeEntries];     // delta at the split
-	__shared__ uint8_t rleft[kMergeEntries];     // the child is the left one
-	__shared__ uint4 front[kSlots];
-	__shared__ uint32_t nfront;
+                                       uint32_t *__restrict__ status, int n,
+                                       PackOut pk = PackOut{}) {
+	__shared__ ClimbShared<kMergeEntries> sh;
+	__shared__ uint32_t pos[kMergeEntries + 1];
+	constexpr int kPer = kMergeEntries / kMergeThreads;
+	static_assert(kMergeFan <= kWave, "group counts in one wave");
 	const int t = threadIdx.x;
-	for (int i = t; i < kTable; i += blockDim.x) table[i] = kEmpty;
-	// the groups' entry counts, one load per thread
-	if (t < ng) gcount[t] = min(in_counts[t], (uint32_t)kSlots);
-	if (t == 0) nfront = 0;
-	__syncthreads();
-	const uint32_t leaf0 = (uint32_t)(n - 1);
-	auto push = [&](const uint4 &e) {
-		const uint32_t slot = atomicAdd(&nfront, 1u);
-		if (out_slots && slot < (uint32_t)kSlots) front[slot] = e;
-		else atomicOr(status, (uint32_t)RTA_LBVH_FRONTIER_OVERFLOW);
-	};
-	uint32_t total = 0;
-	for (int k = 0; k < ng; ++k) total += gcount[k];
-	for (uint32_t ei = (uint32_t)t; ei < total; ei += kMergeThreads) {
-		// entry ei: group g, position ei - before
+	// every wave finds the groups' first items by itself
+	const int lane = __lane_id();
+	const uint32_t mine = lane < ng ? min(in_counts[lane], (uint32_t)kSlots) : 0u;
+	uint32_t upto = mine;
+	for (int off = 1; off < kMergeFan; off <<= 1) {
+		const uint32_t y = __shfl_up(upto, off);
+		if (lane >= off) upto += y;
+	}
+	const int items = (int)__shfl(upto, kMergeFan - 1);
+	const uint32_t first = upto - mine;
+	ClimbItem it[kPer];
+#pragma unroll
+	for (int k = 0; k < kPer; ++k) {
+		const int i = t + k * kMergeThreads;
+		sh.visit[i] = 0;
+		// the last group that starts at or before item i
 		int g = 0;
-		uint32_t before = 0;
-		while (ei >= before + gcount[g]) before += gcount[g++];
-		const uint4 e = in_slots[(size_t)g * kSlots + (ei - before)];
-		ClimbNode c;
-		c.l = e.y;
-		c.r = e.z;
-		c.dl = (int)(e.w & 0xffu) - 1;
-		c.dr = (int)((e.w >> 8) & 0xffu) - 1;
-		{
-			const rta_node nd = nodes[e.x];
-			c.box = nd.box;
-			node_state(make_uint2(nd.type_left_elems, nd.right_tris), c.elems, c.tris);
-		}
-		for (int level = 0; level < 128; ++level) {
-			if (c.dl < 0 && c.dr < 0) break;   // the root of the mesh
-			const bool left = is_left_child(c);
-			const uint32_t s = left ? c.r : c.l - 1u;
-			if (s < lo || s + 1u >= hi) {
-				push(frontier_entry(c, leaf0));
-				break;
+		for (int step = kMergeFan / 2; step > 0; step >>= 1)
+			if (__shfl(first, g + step) <= (uint32_t)i && g + step < ng) g += step;
+		const uint32_t before = __shfl(first, g);
+		if (i < items) {
+			const uint4 e = in_slots[(size_t)g * kSlots + ((uint32_t)i - before)];
+			pos[i] = e.y;
+			sh.delta[i] = (int8_t)((int)(e.w & 0xffu) - 1);
+			if (i == items - 1) {
+				pos[items] = e.z + 1u;
+				sh.delta[items] = (int8_t)((int)((e.w >> 8) & 0xffu) - 1);
 			}
-			const uint32_t r = ei;
-			rbox[0][r] = c.box.min.x; rbox[1][r] = c.box.min.y; rbox[2][r] = c.box.min.z;
-			rbox[3][r] = c.box.max.x; rbox[4][r] = c.box.max.y; rbox[5][r] = c.box.max.z;
-			rfar[r] = left ? c.l : c.r;
-			rdfar[r] = (int8_t)(left ? c.dl : c.dr);
-			rdnear[r] = (int8_t)(left ? c.dr : c.dl);
-			relems[r] = c.elems;
-			rtris[r] = c.tris;
-			rleft[r] = left ? 1u : 0u;
-			// LDS only (the node stores need not wait): the record before
-			// the claim, the sibling's record after
-			__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-			const uint64_t mine = ((uint64_t)s << 32) | (r + 1u);
-			uint32_t h = (s * 2654435761u) >> (32 - kTableBits);
-			uint64_t prev;
-			while (true) {
-				prev = atomicCAS(&table[h], kEmpty, mine);
-				if (prev == kEmpty || (uint32_t)(prev >> 32) == s) break;
-				h = (h + 1u) & (kTable - 1);
-			}
-			if (prev == kEmpty) break;   // the sibling forms the parent
-			__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-			const uint32_t q = (uint32_t)prev - 1u;
-			const int ds = left ? c.dr : c.dl;   // delta(s)
-			ClimbNode sib;
-			sib.box.min = {rbox[0][q], rbox[1][q], rbox[2][q]};
-			sib.box.max = {rbox[3][q], rbox[4][q], rbox[5][q]};
-			sib.elems = relems[q];
-			sib.tris = rtris[q];
-			if (left) { sib.l = s + 1u; sib.r = rfar[q]; sib.dl = ds; sib.dr = rdfar[q]; }
-			else { sib.l = rfar[q]; sib.r = s; sib.dl = rdfar[q]; sib.dr = ds; }
-			if (sib.l < lo || sib.r >= hi || sib.l > sib.r) {
-				// cannot happen for sorted codes; guards the writes below
-				atomicOr(status, (uint32_t)RTA_LBVH_FRONTIER_OVERFLOW);
-				table[h] = ((uint64_t)s << 32) | kFormed;
-				break;
-			}
-			uint32_t x;
-			c = left ? form_parent(c, sib, s, leaf0, nodes, ranges, pk, x)
-			         : form_parent(sib, c, s, leaf0, nodes, ranges, pk, x);
-			table[h] = ((uint64_t)s << 32) |
-			           (pk.pairs && c.elems == kStateInner ? kFormedInner | x : kFormed);
+			it[k].inner = (e.w & kEntryInner) != 0u;
+			it[k].box = nodes[e.x].box;
 		}
 	}
 	__syncthreads();
-	// Per table entry: a single arrival at a split (the sibling lies beyond
-	// [lo, hi)) joins the frontier; an inner node formed here gets its pair
-	// record from the finished nodes (written by this block's threads before
-	// the barrier; inside the climb their stores held it up).
-	// The thread's kPer entries are taken together, so that the node loads
-	// of its pair records (links, then both children) are in flight at once.
-	constexpr int kPer = kTable / kMergeThreads;
-	static_assert(kTable % kMergeThreads == 0, "whole table entries per thread");
-	uint32_t xs[kPer];
-	bool inner[kPer];
-	#pragma unroll
 	for (int k = 0; k < kPer; ++k) {
-		const uint64_t e = table[t + k * kMergeThreads];
-		const uint32_t word = (uint32_t)e;
-		inner[k] = e != kEmpty && word != kFormed && (word & kFormedInner);
-		xs[k] = word & ~kFormedInner;
-		if (e == kEmpty || word == kFormed || (word & kFormedInner)) continue;
-		const uint32_t q = word - 1u, s = (uint32_t)(e >> 32);
-		const int ds = rdnear[q];
-		ClimbNode w;
-		if (rleft[q]) { w.l = rfar[q]; w.r = s; w.dl = rdfar[q]; w.dr = ds; }
-		else { w.l = s + 1u; w.r = rfar[q]; w.dl = ds; w.dr = rdfar[q]; }
-		push(frontier_entry(w, leaf0));
+		const int i = t + k * kMergeThreads;
+		if (i < items) climb(sh, i, items, it[k]);
 	}
-	uint2 links[kPer];
-	#pragma unroll
-	for (int k = 0; k < kPer; ++k)
-		if (inner[k]) links[k] = *reinterpret_cast<const uint2 *>(&nodes[xs[k]]);
-	rta_node nl[kPer], nr[kPer];
-	#pragma unroll
-	for (int k = 0; k < kPer; ++k)
-		if (inner[k]) {
-			nl[k] = nodes[links[k].x >> 1];
-			nr[k] = nodes[links[k].y];
-		}
-	bool slow = false;
-	#pragma unroll
-	for (int k = 0; k < kPer; ++k) {
-		if (!inner[k]) continue;
-		const uint32_t L = links[k].x >> 1, R = links[k].y;
-		const uint32_t lw = link_inner(nl[k].type_left_elems) ? (L << 1) | 1u : nl[k].right_tris << 1;
-		const uint32_t rw = link_inner(nr[k].type_left_elems) ? (R << 1) | 1u : nr[k].right_tris << 1;
-		if (!write_pair(pk.pairs, xs[k], nl[k].box, nr[k].box, lw, rw, L, R)) slow = true;
-	}
-	if (slow && pk.flags) atomicOr(pk.flags, 1u);
 	__syncthreads();
-	const uint32_t nf = min(nfront, (uint32_t)kSlots);
-	if (out_slots && (uint32_t)t < nf) out_slots[t] = front[t];
-	if (out_count && t == 0) *out_count = nf;
+	const uint32_t total = emit_nodes<kMergeEntries, kMergeThreads>(
+	    sh, items, [&](int i) { return pos[i]; }, nodes, ranges, out_slots, n, pk);
+	if (t == 0) {
+		if (total > (out_slots ? (uint32_t)kSlots : 0u))
+			atomicOr(status, (uint32_t)RTA_LBVH_FRONTIER_OVERFLOW);
+		if (out_count) *out_count = min(total, (uint32_t)kSlots);
+	}
 }
 
 // -------------------------------------------------- stage 7: permute
