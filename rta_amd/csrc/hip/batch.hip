@@ -4,8 +4,8 @@
 // (lbvh_body.hpp), so each mesh's nodes, indices and reordered triangles are
 // byte-identical to a build of that mesh alone.
 //
-// Sort: four 8-bit passes over the codes carrying (mesh << 24 | local index),
-// then one pass over that payload's mesh byte carrying the codes.  Both are
+// Sort: three 10-bit passes over the codes carrying (mesh << 24 | local
+// index), then one pass by that payload's mesh byte.  All are
 // stable, so the result is every mesh's own stable sort by code, meshes in
 // order (hence at most 256 meshes and 2^24 triangles per mesh in a batch).
 #include "internal.hpp"
@@ -52,12 +52,6 @@ __global__ __launch_bounds__(256) void batch_morton_kernel(
 	codes[m.tri_off + i] = code;
 	payload[m.tri_off + i] = (it.mesh << 24) | (uint32_t)i;
 	if (code == 0u && status) atomicOr(status, (uint32_t)RTA_LBVH_CODE_ZERO);
-}
-
-__global__ __launch_bounds__(256) void batch_local_index_kernel(uint32_t *__restrict__ idx,
-                                                                long long n) {
-	const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-	if (i < n) idx[i] &= 0xffffffu;
 }
 
 // The traversal layout of one mesh of the batch (pairs, tri4 and flags
@@ -348,13 +342,15 @@ static int batch_build(const char *name, rta_batch b, rta_triangle *tris, rta_no
 	                   items + p.tri_blocks_off, p.d_meshes, w.codes, indices, w.centers, w.bounds,
 	                   status);
 	RTA_LAUNCH_CHECK("batch_morton_kernel");
-	int rc = radix_sort_pairs(w.codes, indices, N, 0, 4, w.sort_work, w.sort_bytes, st);
+	// three passes over the codes, one over the payload's mesh byte, which
+	// also strips that byte; the even number ends in codes/indices
+	uint32_t *ak, *av;
+	radix_alt_buffers(w.sort_work, N, &ak, &av);
+	int rc = radix_pass(w.codes, indices, ak, av, N, 0, 10, false, ~0u, w.sort_work, st);
+	if (rc == RTA_OK) rc = radix_pass(ak, av, w.codes, indices, N, 10, 10, false, ~0u, w.sort_work, st);
+	if (rc == RTA_OK) rc = radix_pass(w.codes, indices, ak, av, N, 20, 10, false, ~0u, w.sort_work, st);
+	if (rc == RTA_OK) rc = radix_pass(ak, av, w.codes, indices, N, 24, 8, true, 0xffffffu, w.sort_work, st);
 	if (rc != RTA_OK) return rc;
-	rc = radix_sort_pairs(indices, w.codes, N, 24, 1, w.sort_work, w.sort_bytes, st);
-	if (rc != RTA_OK) return rc;
-	hipLaunchKernelGGL(batch_local_index_kernel, dim3(grid_for(N, 256)), dim3(256), 0, st,
-	                   indices, (long long)N);
-	RTA_LAUNCH_CHECK("batch_local_index_kernel");
 	auto permute = [&]() -> int {
 		hipLaunchKernelGGL(batch_permute_kernel, dim3((unsigned)p.tri_blocks), dim3(256), 0, st,
 		                   items + p.tri_blocks_off, p.d_meshes, tris, w.scratch, indices, tri4);

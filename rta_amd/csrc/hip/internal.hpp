@@ -8,12 +8,17 @@
 
 namespace rta_hip {
 
-// Stable LSD radix sort of (keys, vals) by `passes` 8-bit digits starting at
-// bit `first_shift` of the key; the result is left in keys/vals.  work:
-// radix_work_bytes(n).
+// Stable LSD radix sort (radix_sort.hip) with work of radix_work_bytes(n):
+// a second pair of buffers and the histograms.
 size_t radix_work_bytes(int n);
-int radix_sort_pairs(uint32_t *keys, uint32_t *vals, int n, int first_shift, int passes,
-                     void *work, size_t work_bytes, hipStream_t st);
+void radix_alt_buffers(void *work, int n, uint32_t **keys, uint32_t **vals);
+// One pass by bits [shift, shift + bits) (bits <= 10) of the key, or of the
+// payload; the payload is stored & keep.
+int radix_pass(const uint32_t *kin, const uint32_t *vin, uint32_t *kout, uint32_t *vout, int n,
+               int shift, int bits, bool of_val, uint32_t keep, void *work, hipStream_t st);
+// 30-bit codes and payloads from the work's second buffers, sorted into keys
+// and vals.
+int radix_sort_codes(uint32_t *keys, uint32_t *vals, int n, void *work, hipStream_t st);
 
 // One mesh of a batch as the device sees it.
 struct BatchMesh {

@@ -5,6 +5,7 @@
 // documented at the stage body (lbvh_body.hpp).  This file holds the
 // single-mesh kernels and entry points; batch.hip runs the same bodies for
 // many meshes per launch.
+#include "internal.hpp"
 #include "lbvh_body.hpp"
 
 #include <cstdio>
@@ -497,9 +498,12 @@ static int build_impl(const char *name, rta_triangle *tris, int n, rta_node *nod
 	} else {
 		if (rc == RTA_OK) rc = rta_lbvh_voxel_bounds(w.bounds, w.partials, n, s);
 		mark(2);
-		if (rc == RTA_OK) rc = rta_lbvh_morton_codes(w.codes, indices, w.centers, w.bounds, status, n, s);
+		// into the sort's second buffers: its three passes end in codes/indices
+		uint32_t *keys, *vals;
+		radix_alt_buffers(w.sort_work, n, &keys, &vals);
+		if (rc == RTA_OK) rc = rta_lbvh_morton_codes(keys, vals, w.centers, w.bounds, status, n, s);
 		mark(3);
-		if (rc == RTA_OK) rc = rta_lbvh_sort(w.codes, indices, n, w.sort_work, w.sort_bytes, s);
+		if (rc == RTA_OK) rc = radix_sort_codes(w.codes, indices, n, w.sort_work, as_stream(s));
 	}
 	mark(4);
 	// the hierarchy is emitted by the bottom-up stage: no pass of its own
