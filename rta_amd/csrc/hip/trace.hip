@@ -742,7 +742,7 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
     uint32_t *__restrict__ err, uint32_t *__restrict__ queue, int refill_min, int steps,
     int leaf_min, const BatchMesh *__restrict__ meshes, int n_meshes,
     const uint32_t *__restrict__ root_words, uint32_t *__restrict__ ovf,
-    const uint32_t *__restrict__ ray_list, SeedArgs seed) {
+    const uint32_t *__restrict__ ray_list, SeedArgs seed, int fixed_rays) {
 	static_assert(!SEEDED || (!ANY_HIT && !BATCHED), "seeding: closest hit on one mesh");
 	static_assert(STACK >= kRows && STACK <= kStack, "kRows to kStack entries");
 	// Row r of the stack holds one word per lane.  The top entry lives in a
@@ -796,6 +796,12 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 	// 1,621 us, then 1,623 / 1,661 / 1,963; bounce rays 1,568, then 1,551 /
 	// 1,539 / 1,694), so one mesh takes 1/4 and a batch 1/2.
 	uint32_t run_at = 0, run_end = 0, left = n;
+	// With fixed_rays the wave's only run is its own, without the queue.
+	if (fixed_rays) {
+		run_at = min((blockIdx.x * (BLOCK / kWave) + (uint32_t)wave) * (uint32_t)fixed_rays, n);
+		run_end = min(run_at + (uint32_t)fixed_rays, n);
+		exhausted = true;
+	}
 	const uint32_t split = (BATCHED ? 2u : 4u) * gridDim.x * (BLOCK / kWave);
 	const int share = 32 - __builtin_clz(split);
 	// BATCHED: the last refill's mesh and its rays
@@ -1353,19 +1359,39 @@ int launch_persistent(const float *tri4, const rta_node_pair *pairs, const uint3
 	}
 	const int bpc = blocks_per_cu > 0 ? blocks_per_cu : occ[dev];
 	const long long want = (long long)cus[dev] * bpc;
-	const long long need = ((long long)n_rays + BLOCK - 1) / BLOCK;
+	long long need = ((long long)n_rays + BLOCK - 1) / BLOCK;
+	// Rays that are all in flight at once need no queue: each wave has its own
+	// (640 x 360 primary rays of the 2.3 M-triangle terrain 381 -> 343 us,
+	// bounce rays 335 -> 285 us).  Half-filled waves end sooner, as their rays
+	// diverge less, and while all of them fit they cost nothing (500 x 300
+	// rays, 64 then 32 a wave: 353 / 310 -> 336 / 297 us); quarters are worse
+	// once a SIMD has to run two (200 x 150 bounce rays of a 90 k-triangle
+	// terrain, 64, 32 and 16 a wave: 166, 159, 166 us) and better before that
+	// (128 x 128: 157, 162, 150 us); eighths gain nothing over quarters.
+	int fixed_rays = 0;
+	if (need <= want) {
+		constexpr int kWaves = BLOCK / kWave;
+		auto blocks_of = [&](int rays) { return ((long long)n_rays + rays * kWaves - 1) / (rays * kWaves); };
+		fixed_rays = kWave;
+		if (blocks_of(kWave / 2) <= want) fixed_rays = kWave / 2;
+		if (blocks_of(kWave / 4) <= want && blocks_of(kWave / 4) * kWaves <= 4LL * cus[dev])
+			fixed_rays = kWave / 4;
+		need = blocks_of(fixed_rays);
+	}
 	const unsigned blocks = (unsigned)(want < need ? want : need);
 	if (STACK < kStack) {
 		const int rc = rta_hip_fill_u32(ovf, 0u, 1, reinterpret_cast<rta_stream>(st));
 		if (rc != RTA_OK) return rc;
 	}
-	hipLaunchKernelGGL(fill_queue_kernel, dim3(1), dim3(64), 0, st, queue);
-	RTA_LAUNCH_CHECK("fill_queue_kernel");
+	if (!fixed_rays) {
+		hipLaunchKernelGGL(fill_queue_kernel, dim3(1), dim3(64), 0, st, queue);
+		RTA_LAUNCH_CHECK("fill_queue_kernel");
+	}
 	hipLaunchKernelGGL((trace_cis_persistent_kernel<BLOCK, ANY_HIT, BATCHED, SEEDED, STACK>),
 	                   dim3(blocks), dim3(BLOCK), 0, st, (const float4 *)tri4,
 	                   (const float4 *)pairs, flags, root_word, ro, rd, rmax, n_rays, ray_count,
 	                   hits, err, queue, refill_min, steps, leaf_min, meshes, n_meshes,
-	                   root_words, STACK < kStack ? ovf : nullptr, ray_list, seed);
+	                   root_words, STACK < kStack ? ovf : nullptr, ray_list, seed, fixed_rays);
 	RTA_LAUNCH_CHECK("trace_cis_persistent_kernel");
 	if (STACK < kStack)
 		return launch_persistent<BLOCK, ANY_HIT, BATCHED, SEEDED, kStack>(

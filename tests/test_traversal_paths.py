@@ -98,6 +98,22 @@ def test_every_stack_depth(gpu, shuffled, shadow, stack, block):
         assert int(ovf.download(np.uint32, 1)[0]) == int((depth > stack).sum())
 
 
+# 16, 32 or 64 rays a wave without a queue, or waves that share one: the
+# largest launch of each and the next, on a chip of 256 CUs with 20 waves each
+@pytest.mark.gpu
+@pytest.mark.parametrize("shadow", [False, True])
+@pytest.mark.parametrize("n", [1, 17, 16384, 16385, 163840, 163841, 327680, 327681])
+def test_rays_per_wave(gpu, n, shadow):
+    tris, nodes = forest()
+    o, d, t = forest_rays(True)
+    exp, _ = oracle.trace_kernel(tris, nodes, o, d, t, any_hit=shadow)
+    at = np.arange(n) % len(t)
+    o, d = (np.ascontiguousarray(a.reshape(-1, 3)[at]).reshape(-1) for a in (o, d))
+    got = Packed(tris, nodes).trace(DeviceBuffer.from_array(o), DeviceBuffer.from_array(d),
+                                    DeviceBuffer.from_array(t[at]), n, 32, shadow=shadow)
+    assert same_records(got, exp[at])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("axis", [0, 1, 2])
 def test_boxes_with_min_above_max(gpu, axis):
