@@ -488,7 +488,16 @@ __global__ __launch_bounds__(256) void store_params_kernel(uint16_t *__restrict_
 // treelet for positive logits), kept in a sorted register quadruple by one
 // max and three med3 per key, and the four lanes of a ray merged by
 // shuffles at the end.
-
+//
+// What bounds it: instruction issue of the selection and, per 32 rays, the
+// latency of loads and products with four waves a SIMD (the LDS copy of
+// layer 4 allows no more).  2.06 M rays, top-4: 542 us with every key
+// inserted (4 instructions each) and the hidden layers' weights read from
+// the caches, whose 32 KB a tile kept missing L1; 502 with one insertion per
+// four keys as a rule (13 instructions per four instead of 21; four keys of
+// one tile: 540), 485 with three quarters of those weights in LDS, 476 with
+// half of the next round's operands read ahead.  The products and LDS reads
+// alone take 128 us, the encoding and hidden layers alone 139 (188 before).
 constexpr int kInferWaves = 16;                       // 1024 threads per block
 
 __device__ inline unsigned bf16x2(float a, float b) {
@@ -501,11 +510,11 @@ __device__ inline v4f mfma32(v4u a, v4u b, v4f c) {
 }
 
 // one 64-wide ReLU layer for NS sets of 16 rays; in: KS k-steps of B
-// operands per set, out: the next layer's 2 k-steps per set
-template <int KS, int NS>
-__device__ inline void hidden_layer(v4u out[NS][2], const v4u in[NS][KS],
-                                    const v4u *__restrict__ wp, const float *__restrict__ bias,
-                                    int lane) {
+// operands per set, out: the next layer's 2 k-steps per set; record(k): the
+// lane's k-th weight record
+template <int KS, int NS, class Record>
+__device__ inline void hidden_layer(v4u out[NS][2], const v4u in[NS][KS], Record record,
+                                    const float *__restrict__ bias, int lane) {
 	unsigned d[NS][4][2];
 	#pragma unroll
 	for (int t = 0; t < 4; ++t) {
@@ -515,7 +524,7 @@ __device__ inline void hidden_layer(v4u out[NS][2], const v4u in[NS][KS],
 		for (int r = 0; r < NS; ++r) a[r] = (v4f){b.x, b.y, b.z, b.w};
 		#pragma unroll
 		for (int s = 0; s < KS; ++s) {
-			const v4u w = wp[(t * KS + s) * 64 + lane];
+			const v4u w = record(t * KS + s);
 			#pragma unroll
 			for (int r = 0; r < NS; ++r) a[r] = mfma32(w, in[r][s], a[r]);
 		}
@@ -567,14 +576,31 @@ __device__ inline void insert4(float t[4], float x) {
 	t[0] = n0; t[1] = n1; t[2] = n2; t[3] = n3;
 }
 
+// the largest v and the smallest w of a ray's four lanes (lanes 16 apart)
+__device__ inline void ray_max_min(float &v, float &w) {
+	const unsigned vb = __float_as_uint(v), wb = __float_as_uint(w);
+	const auto v16 = __builtin_amdgcn_permlane16_swap(vb, vb, false, false);
+	const auto w16 = __builtin_amdgcn_permlane16_swap(wb, wb, false, false);
+	const unsigned v2 = __float_as_uint(fmaxf(__uint_as_float(v16[0]), __uint_as_float(v16[1])));
+	const unsigned w2 = __float_as_uint(fminf(__uint_as_float(w16[0]), __uint_as_float(w16[1])));
+	const auto v32 = __builtin_amdgcn_permlane32_swap(v2, v2, false, false);
+	const auto w32 = __builtin_amdgcn_permlane32_swap(w2, w2, false, false);
+	v = fmaxf(__uint_as_float(v32[0]), __uint_as_float(v32[1]));
+	w = fminf(__uint_as_float(w32[0]), __uint_as_float(w32[1]));
+}
+
 __device__ inline int key_cluster(float k) { return 1023 - (int)(__float_as_uint(k) & 0x3ffu); }
 
 // Persistent: each wave takes tiles of 32 rays (two sets of 16) from a
-// static stride; layer 4's permuted weights (133,120 B) and biases sit in
-// LDS, one block of 16 waves per CU.  LOGITS: also write every output (for
-// testing; a separate instance keeps the stores out of the fast loop).  K:
-// 4, or 1 (top-1 only: one max per key; entries 1..3 of a ray's top are
-// written as -1).
+// static stride; the biases and the permuted weights of layers 4, 3 and 2
+// and half of layer 1 sit in LDS (162,624 B), one block of 16 waves per CU.
+// LOGITS: also write every output (for testing; a separate instance keeps
+// the stores out of the fast loop).  K: 4, or 1 (top-1 only: entries 1..3 of
+// a ray's top are written as -1).
+//
+// A tile whose logits could overflow to infinity (`wild`: a weight, bias or
+// activation of layer 4 beyond 2^34, 2^66 or 2^65) inserts its keys one by
+// one, in treelet order: such keys are NaNs and their order matters.
 template <bool LOGITS, int K>
 __global__ __launch_bounds__(1024) void infer_kernel(const v4u *__restrict__ wp,
                                                      const float *__restrict__ params,
@@ -586,76 +612,201 @@ __global__ __launch_bounds__(1024) void infer_kernel(const v4u *__restrict__ wp,
                                                      float *__restrict__ logits) {
 	__shared__ v4u w4s[kRec4];
 	__shared__ v4f b4s[kOutP / 4];
-	for (int i = threadIdx.x; i < kRec4; i += kInferWaves * kWave) w4s[i] = wp[pW4 + i];
-	for (int i = threadIdx.x; i < kOutP / 4; i += kInferWaves * kWave)
-		b4s[i] = reinterpret_cast<const v4f *>(params + oB4)[i];
-	__syncthreads();
+	__shared__ v4u w1s[8 * kWave], w23s[16 * kWave];
+	__shared__ float bs[3 * kHid];
+	for (int i = threadIdx.x; i < 8 * kWave; i += kInferWaves * kWave) {
+		w1s[i] = wp[pW1 + i];
+		w23s[i] = wp[pW2 + i];
+		w23s[8 * kWave + i] = wp[pW3 + i];
+	}
+	if (threadIdx.x < kHid) {
+		bs[threadIdx.x] = params[oB1 + threadIdx.x];
+		bs[kHid + threadIdx.x] = params[oB2 + threadIdx.x];
+		bs[2 * kHid + threadIdx.x] = params[oB3 + threadIdx.x];
+	}
+	int big = 0;   // a weight >= 2^34 or a bias >= 2^66
+	for (int i = threadIdx.x; i < kRec4; i += kInferWaves * kWave) {
+		const v4u w = wp[pW4 + i];
+		w4s[i] = w;
+		#pragma unroll
+		for (int k = 0; k < 4; ++k)
+			big |= (w[k] & 0x7fffu) >= 0x5080u || (w[k] & 0x7fff0000u) >= 0x50800000u;
+	}
+	for (int i = threadIdx.x; i < kOutP / 4; i += kInferWaves * kWave) {
+		const v4f b = reinterpret_cast<const v4f *>(params + oB4)[i];
+		b4s[i] = b;
+		#pragma unroll
+		for (int k = 0; k < 4; ++k) big |= (__float_as_uint(b[k]) & 0x7fffffffu) >= 0x60800000u;
+	}
+	const bool big_weights = __syncthreads_or(big) != 0;
 	const int lane = __lane_id(), g = lane >> 4, col = lane & 15;
 	const int n_tiles = (n + 31) / 32;
+	unsigned mask = 0xfffffc00u;
+	asm("" : "+v"(mask));   // in a register: and_or takes one scalar operand
 	for (int tile = blockIdx.x * kInferWaves + (int)(threadIdx.x / kWave); tile < n_tiles;
 	     tile += gridDim.x * kInferWaves) {
 		v4u x[2][4];
 		#pragma unroll
 		for (int r = 0; r < 2; ++r) encode_operands(x[r], ro, rd, tile * 32 + r * 16 + col, n, lo, scale, g);
-		// the hidden layers' weights and biases are loaded per tile (from the
-		// caches): the empty asm hides their loop invariance, which would
+		// the hidden layers' weights and biases are loaded per tile: the empty asm hides their loop invariance, which would
 		// otherwise hoist all of them into registers and spill (an opaque
 		// offset, so that the loads stay global rather than flat)
 		int z = 0;
 		asm volatile("" : "+s"(z));
 		const v4u *wq = wp + z;
-		const float *pq = params + z;
 		v4u h1[2][2], h2[2][2], h3[2][2];
-		hidden_layer<4, 2>(h1, x, wq + pW1, pq + oB1, lane);
-		hidden_layer<2, 2>(h2, h1, wq + pW2, pq + oB2, lane);
-		hidden_layer<2, 2>(h3, h2, wq + pW3, pq + oB3, lane);
-		// layer 4: 64 treelet tiles into the running top-4 of each lane,
-		// software-pipelined: the products of tile t+1 are issued and the
-		// operands of tile t+2 fetched before the keys of tile t are inserted;
-		// tile 64 (the log distance and padding) comes out of the last round
+		const float *bq = bs + z;
+		auto w1 = [&](int k) { return k < 8 ? w1s[z + k * kWave + lane] : wq[pW1 + k * kWave + lane]; };
+		auto w2 = [&](int k) { return w23s[z + k * kWave + lane]; };
+		auto w3 = [&](int k) { return w23s[z + (8 + k) * kWave + lane]; };
+		hidden_layer<4, 2>(h1, x, w1, bq, lane);
+		hidden_layer<2, 2>(h2, h1, w2, bq + kHid, lane);
+		hidden_layer<2, 2>(h3, h2, w3, bq + 2 * kHid, lane);
 		float tk[2][4];
 		#pragma unroll
 		for (int r = 0; r < 2; ++r)
 			#pragma unroll
 			for (int i = 0; i < 4; ++i) tk[r][i] = -__builtin_inff();
-		const unsigned low0 = 1023u - 4u * (unsigned)g;
-		v4u w0 = w4s[lane], w1 = w4s[64 + lane];
-		v4f bias = b4s[g];
-		v4f acc[2];
-		acc[0] = mfma32(w1, h3[0][1], mfma32(w0, h3[0][0], bias));
-		acc[1] = mfma32(w1, h3[1][1], mfma32(w0, h3[1][0], bias));
-		w0 = w4s[2 * 64 + lane];
-		w1 = w4s[3 * 64 + lane];
-		bias = b4s[4 + g];
-#pragma unroll 1
-		for (int t = 0; t < kClusters / 16; ++t) {
-			v4f nxt[2];
-			nxt[0] = mfma32(w1, h3[0][1], mfma32(w0, h3[0][0], bias));
-			nxt[1] = mfma32(w1, h3[1][1], mfma32(w0, h3[1][0], bias));
-			const int u = t + 2 < kOutP / 16 ? t + 2 : kOutP / 16 - 1;
-			w0 = w4s[(2 * u) * 64 + lane];
-			w1 = w4s[(2 * u + 1) * 64 + lane];
-			bias = b4s[4 * u + g];
+		// largest operand of layer 4, as bf16 bits (>= 0: ReLU)
+		typedef short v2s __attribute__((ext_vector_type(2)));
+		v2s hmax = {0, 0};
+		#pragma unroll
+		for (int r = 0; r < 2; ++r)
 			#pragma unroll
-			for (int r = 0; r < 2; ++r)
+			for (int q = 0; q < 8; ++q)
+				hmax = __builtin_elementwise_max(hmax, __builtin_bit_cast(v2s, h3[r][q >> 2][q & 3]));
+		const bool wild = big_weights ||
+		                  __builtin_amdgcn_ballot_w64(hmax.x >= 0x6080 || hmax.y >= 0x6080) != 0ull;
+		v4f acc[2];
+		if (!wild) {
+			// Four keys of a lane at a time, from tiles u + 16k: treelets that
+			// lie 256 apart and rarely are a ray's best together (neighbours,
+			// as one tile's four, often are).  Their largest is inserted and,
+			// where some lane's second could be among its four best, all are.
+			struct Tile { v4u w0, w1; v4f bias; };
+			auto load = [&](int t) {
+				return Tile{w4s[(2 * t) * 64 + lane], w4s[(2 * t + 1) * 64 + lane], b4s[4 * t + g]};
+			};
+			constexpr int kAhead = 2;   // tiles of the next round read during this one
+			Tile ahead[kAhead];
+			#pragma unroll
+			for (int k = 0; k < kAhead; ++k) ahead[k] = load(16 * k);
+#pragma unroll 1
+			for (int u = 0; u < kClusters / 64; ++u) {
+				v4f a[2][4];
+				Tile here[4];
 				#pragma unroll
-				for (int i = 0; i < 4; ++i) {
-					const unsigned low = low0 - 16u * (unsigned)t - (unsigned)i;
-					const float key = __uint_as_float((__float_as_uint(acc[r][i]) & 0xfffffc00u) | low);
-					if (K == 1) tk[r][0] = fmaxf(tk[r][0], key);
-					else insert4(tk[r], key);
-				}
-			if (LOGITS)
+				for (int k = 0; k < 4; ++k) here[k] = k < kAhead ? ahead[k] : load(u + 16 * k);
 				#pragma unroll
-				for (int r = 0; r < 2; ++r) {
-					const int ray = tile * 32 + r * 16 + col;
-					if (ray < n)
+				for (int k = 0; k < 4; ++k)
+					#pragma unroll
+					for (int r = 0; r < 2; ++r)
+						a[r][k] = mfma32(here[k].w1, h3[r][1], mfma32(here[k].w0, h3[r][0], here[k].bias));
+				#pragma unroll
+				for (int k = 0; k < kAhead; ++k) ahead[k] = load(u + 1 + 16 * k);
+				#pragma unroll
+				for (int r = 0; r < 2; ++r)
+					#pragma unroll
+					for (int i = 0; i < 4; ++i) {
+						float key[4];
 						#pragma unroll
-						for (int i = 0; i < 4; ++i)
-							logits[(size_t)ray * kOutP + 16 * t + 4 * g + i] = acc[r][i];
-				}
-			acc[0] = nxt[0];
-			acc[1] = nxt[1];
+						for (int k = 0; k < 4; ++k)
+							key[k] = __uint_as_float((__float_as_uint(a[r][k][i]) & mask) |
+							                         (unsigned)(1011 - 16 * (u + 16 * k) - i));
+						const float top3 = fmaxf(fmaxf(key[0], key[1]), key[2]);
+						if (K == 1) {
+							tk[r][0] = fmaxf(fmaxf(tk[r][0], top3), key[3]);
+							continue;
+						}
+						const float second = __builtin_amdgcn_fmed3f(
+						    top3, __builtin_amdgcn_fmed3f(key[0], key[1], key[2]), key[3]);
+						if (__builtin_amdgcn_ballot_w64(second > tk[r][3]) != 0ull) {
+							#pragma unroll
+							for (int k = 0; k < 4; ++k) insert4(tk[r], key[k]);
+						} else {
+							insert4(tk[r], fmaxf(top3, key[3]));
+						}
+					}
+				if (LOGITS)
+					#pragma unroll
+					for (int r = 0; r < 2; ++r) {
+						const int ray = tile * 32 + r * 16 + col;
+						if (ray < n)
+							#pragma unroll
+							for (int k = 0; k < 4; ++k)
+								#pragma unroll
+								for (int i = 0; i < 4; ++i)
+									logits[(size_t)ray * kOutP + 16 * (u + 16 * k) + 4 * g + i] = a[r][k][i];
+					}
+				// After rounds 0, 1, 3, 7 and 15 the ray's four lanes agree on a
+				// bound: a lane's fourth best, or the least of the lanes' bests,
+				// has four keys of the ray at or above it.  Entries below it give
+				// way to a value just under every key with its 13 mantissa bits,
+				// so never one of the ray's best four, and the checks above fail
+				// less.
+				if (K != 1 && (u & (u + 1)) == 0)
+					#pragma unroll
+					for (int r = 0; r < 2; ++r) {
+						float fourth = tk[r][3], first = tk[r][0];
+						ray_max_min(fourth, first);
+						const float t = __uint_as_float(__float_as_uint(fmaxf(fourth, first)) & mask);
+						const float below = __builtin_fmaf(-0x1p-12f, fabsf(t), t) - FLT_MIN;
+						#pragma unroll
+						for (int i = 0; i < 4; ++i) tk[r][i] = fmaxf(tk[r][i], below);
+					}
+			}
+			// the keys' bits of the lane group, which do not change a lane's order
+			#pragma unroll
+			for (int r = 0; r < 2; ++r) {
+				#pragma unroll
+				for (int i = 0; i < (K == 1 ? 1 : 4); ++i)
+					tk[r][i] = __uint_as_float(__float_as_uint(tk[r][i]) | (unsigned)(3 - g) << 2);
+				constexpr int t = kClusters / 16;
+				acc[r] = mfma32(w4s[(2 * t + 1) * 64 + lane], h3[r][1],
+				                mfma32(w4s[(2 * t) * 64 + lane], h3[r][0], b4s[4 * t + g]));
+			}
+		} else {
+			// 64 treelet tiles, key by key: the products of tile t+1 are issued
+			// and the operands of tile t+2 fetched before the keys of tile t are
+			// inserted; tile 64 (the log distance and padding) comes out last
+			const unsigned low0 = 1023u - 4u * (unsigned)g;
+			v4u w0 = w4s[lane], w1 = w4s[64 + lane];
+			v4f bias = b4s[g];
+			acc[0] = mfma32(w1, h3[0][1], mfma32(w0, h3[0][0], bias));
+			acc[1] = mfma32(w1, h3[1][1], mfma32(w0, h3[1][0], bias));
+			w0 = w4s[2 * 64 + lane];
+			w1 = w4s[3 * 64 + lane];
+			bias = b4s[4 + g];
+#pragma unroll 1
+			for (int t = 0; t < kClusters / 16; ++t) {
+				v4f nxt[2];
+				nxt[0] = mfma32(w1, h3[0][1], mfma32(w0, h3[0][0], bias));
+				nxt[1] = mfma32(w1, h3[1][1], mfma32(w0, h3[1][0], bias));
+				const int u = t + 2 < kOutP / 16 ? t + 2 : kOutP / 16 - 1;
+				w0 = w4s[(2 * u) * 64 + lane];
+				w1 = w4s[(2 * u + 1) * 64 + lane];
+				bias = b4s[4 * u + g];
+				#pragma unroll
+				for (int r = 0; r < 2; ++r)
+					#pragma unroll
+					for (int i = 0; i < 4; ++i) {
+						const unsigned low = low0 - 16u * (unsigned)t - (unsigned)i;
+						const float key = __uint_as_float((__float_as_uint(acc[r][i]) & 0xfffffc00u) | low);
+						if (K == 1) tk[r][0] = fmaxf(tk[r][0], key);
+						else insert4(tk[r], key);
+					}
+				if (LOGITS)
+					#pragma unroll
+					for (int r = 0; r < 2; ++r) {
+						const int ray = tile * 32 + r * 16 + col;
+						if (ray < n)
+							#pragma unroll
+							for (int i = 0; i < 4; ++i)
+								logits[(size_t)ray * kOutP + 16 * t + 4 * g + i] = acc[r][i];
+					}
+				acc[0] = nxt[0];
+				acc[1] = nxt[1];
+			}
 		}
 		if (logdist || LOGITS) {
 			const int t = kClusters / 16;
@@ -868,9 +1019,10 @@ __global__ __launch_bounds__(2 * SETS * kWave) void train_rows_kernel(
 		encode_operands(xs[0], ro, rd, act ? ray : n, n, lo, scale, g);
 		const float *pq = params + z;
 		v4u h1[1][2], h2[1][2], h3[1][2];
-		hidden_layer<4, 1>(h1, xs, wq + pW1, pq + oB1, lane);
-		hidden_layer<2, 1>(h2, h1, wq + pW2, pq + oB2, lane);
-		hidden_layer<2, 1>(h3, h2, wq + pW3, pq + oB3, lane);
+		const v4u *wq1 = wq + pW1, *wq2 = wq + pW2, *wq3 = wq + pW3;
+		hidden_layer<4, 1>(h1, xs, [&](int k) { return wq1[k * kWave + lane]; }, pq + oB1, lane);
+		hidden_layer<2, 1>(h2, h1, [&](int k) { return wq2[k * kWave + lane]; }, pq + oB2, lane);
+		hidden_layer<2, 1>(h3, h2, [&](int k) { return wq3[k * kWave + lane]; }, pq + oB3, lane);
 		if (base == blockIdx.x * SETS) {                  // W4 and its bias in LDS
 			__builtin_amdgcn_s_waitcnt(0);
 			__syncthreads();

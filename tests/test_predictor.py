@@ -202,6 +202,55 @@ def test_infer_matches_reference(gpu):
     assert np.all(t1[:, 1:] == -1)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("top_k", [1, 4])
+@pytest.mark.parametrize("case", ["equal", "rising", "falling", "negative", "one_quad", "one_tile",
+                                  "around_zero", "large", "random"])
+def test_infer_selection(gpu, case, top_k):
+    """The selection against the key rule on the kernel's own logits, for
+    logits that stand in every order, sign and place: layer 4 is its biases
+    (and, for "random" and "large", weights; "large" ones up to 1e13, whose
+    logits are finite)."""
+    n, many = 77, 32 * (4 * 256) + 33     # one wave a SIMD at most, and more
+    rng = np.random.default_rng(23)
+    b = {"equal": np.full(1024, 1.5), "rising": np.arange(1024) / 64.0,
+         "falling": -np.arange(1024) / 64.0, "negative": -1.0 - rng.random(1024),
+         "around_zero": rng.permutation(np.arange(-512, 512)) * 2.0 ** -140,
+         "random": rng.normal(size=1024), "large": rng.normal(size=1024)}.get(case, np.zeros(1024))
+    if case == "one_quad":
+        b[[17, 17 + 256, 17 + 512, 17 + 768]] = [3, 1, 4, 2]
+    if case == "one_tile":
+        b[640:656] = 2.0
+    pred = P.HitPredictor(1024, seed=5, scene_min=LO, scene_max=HI)
+    params = pred.params()
+    w4, b4 = P.LAYOUT["W4"][0], P.LAYOUT["b4"][0]
+    if case not in ("random", "large"):
+        params[w4:w4 + 1040 * 64] = 0.0
+    if case == "large":
+        params[w4:w4 + 1024 * 64] = rng.normal(scale=1e13, size=1024 * 64).astype(np.float32)
+    params[b4:b4 + 1024] = b.astype(np.float32)
+    pred.set_params(params)
+    o, d = _random_rays(n, 29)
+    ob, db = DeviceBuffer.from_array(o), DeviceBuffer.from_array(d)
+    logits, top, top2 = DeviceBuffer(4 * 1040 * n), DeviceBuffer(16 * n), DeviceBuffer(16 * n)
+    pred.infer(ob, db, n, top=top, logits=logits, top_k=top_k)
+    pred.infer(ob, db, n, top=top2, top_k=top_k)
+    rta_amd.synchronize()
+    exp = keyed_top4(logits.download(np.float32, 1040 * n).reshape(n, 1040))
+    if top_k == 1:
+        exp[:, 1:] = -1
+    assert np.array_equal(top.download(np.int32, 4 * n).reshape(n, 4), exp)
+    assert np.array_equal(top2.download(np.int32, 4 * n).reshape(n, 4), exp)
+    at = np.arange(many) % n
+    ob, db = (DeviceBuffer.from_array(np.ascontiguousarray(a.reshape(-1, 3)[at])) for a in (o, d))
+    logits, top, top2 = DeviceBuffer(4160 * many), DeviceBuffer(16 * many), DeviceBuffer(16 * many)
+    pred.infer(ob, db, many, top=top, logits=logits, top_k=top_k)
+    pred.infer(ob, db, many, top=top2, top_k=top_k)
+    rta_amd.synchronize()
+    assert np.array_equal(top.download(np.int32, 4 * many).reshape(many, 4), exp[at])
+    assert np.array_equal(top2.download(np.int32, 4 * many).reshape(many, 4), exp[at])
+
+
 def _sample_index(seed, frame, i, count):
     """rta_pred_sample's draw on the host (splitmix64 finaliser of
     seed * golden + (frame << 32) + i, modulo count)."""
