@@ -846,8 +846,8 @@ def main():
     queue = DeviceBuffer(4)
     tcfg = TraceConfig(args.block, args.refill, args.steps_per_refill, 0, args.leaf_min)
 
-    # the coherent primary rays gain from a short stack's extra resident
-    # waves; the incoherent bounce rays lose L2 hits with them
+    # the primary rays with the short stack, whose overflowing rays (none
+    # here) are traced again; the bounce rays with the reference's depth
     pcfg = TraceConfig(args.block, args.refill, args.steps_per_refill, 0, args.leaf_min,
                        args.primary_stack)
     povf = DeviceBuffer(4 * (R + 1))

@@ -332,18 +332,19 @@ int rta_trace_cis_packed(const float *tri4, const rta_node_pair *pairs,
  * checks), blocks_per_cu (0 = as many as fit) and leaf_min (a wave tests
  * leaf triangles once at least ceil(leaf_min * active / 64) of its active
  * lanes wait at a leaf, or no lane is at an inner node; 1..64, 0 = default
- * 10) and stack (LDS stack entries: 32, the reference's depth, or 16 or 24
- * for a smaller LDS footprint and more resident waves, with an overflow
- * list (the _ovf entry points and the batch API): a ray that would need
- * more is traced again with 32 entries; 0 = 32).  None of these changes a
- * result. */
+ * 10) and stack (the entries a ray may use: 32, the reference's depth, or
+ * 16 or 24 with an overflow list (the _ovf entry points and the batch API):
+ * a ray that would need more is traced again with 32 entries; 0 = 32.  The
+ * kernel's LDS footprint is the same for all three).  None of these changes
+ * a result. */
 typedef struct rta_trace_config {
 	int block, refill_min, steps, blocks_per_cu, leaf_min, stack;
 } rta_trace_config;
 
 /* Persistent form of rta_trace_cis_packed: a machine-filling grid of waves
  * that refill idle lanes from a queue counter (`queue`, one device word of
- * scratch, cleared by this call with a kernel).  Same results, except that
+ * scratch, cleared by this call with a kernel where the rays are more than
+ * are in flight at once and unused otherwise).  Same results, except that
  * a miss only stores t = FLT_MAX and leaves beta, gamma and ref as they
  * were (the reset sentinel).  cfg may be NULL (defaults 64/16/32/0/10). */
 int rta_trace_cis_persistent(const float *tri4, const rta_node_pair *pairs,
@@ -376,15 +377,14 @@ int rta_trace_shadow_cis_persistent(const float *tri4,
                                     uint32_t *queue,
                                     const rta_trace_config *cfg, rta_stream s);
 
-/* The two persistent traversals with a short LDS stack (no counterpart in
+/* The two persistent traversals with a short stack (no counterpart in
  * the reference, whose stack depth is fixed at 32, bbvh-cuda/kernels.cu:
  * 787): with cfg->stack 16 or 24 a ray that would push beyond it is
  * abandoned onto `overflow` (device words: a count, then up to n_rays ray
  * ids; cleared by the call with a kernel) and traced again with 32 entries
  * by a second launch over that list, so every record equals the 32-entry
- * traversal's.  Fewer entries mean more resident waves: coherent rays gain,
- * incoherent ones can lose L2 hits.  With cfg->stack 32 (or cfg NULL) the
- * list is not used; overflow must not be NULL either way. */
+ * traversal's.  With cfg->stack 32 (or cfg NULL) the list is not used;
+ * overflow must not be NULL either way. */
 int rta_trace_cis_persistent_ovf(const float *tri4, const rta_node_pair *pairs,
                                  const uint32_t *flags, uint32_t root_link,
                                  uint32_t root_index, const float *ray_orig,

@@ -608,9 +608,10 @@ __global__ void fill_queue_kernel(uint32_t *queue) {
 
 // Persistent waves: each lane traces one ray at a time; when at least
 // `refill_min` lanes of a wave are idle the wave takes that many new rays
-// (consecutive ids, so they are coherent) from a global queue counter with
-// one atomic.  A wave never waits for another, and it leaves the loop once
-// the queue is exhausted and all of its lanes are idle.
+// (consecutive ids, so they are coherent) from its run, and a new run from a
+// global queue counter with one atomic.  A wave never waits for another, and
+// it leaves the loop once the queue and its run are exhausted and all of its
+// lanes are idle.
 //
 // Each traversal step of the wave is either an inner-node step (every lane
 // standing at an inner node visits it) or a leaf step (every lane standing
@@ -629,9 +630,10 @@ __global__ void fill_queue_kernel(uint32_t *queue) {
 // staged fetch in `run` below; coherent rays the VALU (about 95
 // instructions per wave-step at inner nodes, 116 before the stack's top
 // moved to a register, the decision's masks to scalar registers and the
-// records' stores out of the step).  On the 2.3 M-triangle terrain, 2.07 M
-// rays each: bounce rays 1,917 -> 1,582 us, primary rays 1,826-1,886 ->
-// 1,634 us; shadow rays of a 400 k-triangle terrain (0.88 M) 739 -> 632 us.
+// records' stores out of the step; 96 % of the issue slots, 81 % for bounce
+// rays).  On the 2.3 M-triangle terrain, 2.07 M rays each: bounce rays 1,910
+// -> 1,549 us, primary rays 1,890 -> 1,636 us; shadow rays of a 400
+// k-triangle terrain (0.88 M) 750 -> 640 us.
 //
 // BATCHED: rays of many meshes in one launch.  Ray r belongs to the mesh
 // whose [ray_off, ray_off + n_rays) holds it; that mesh's pair records start
@@ -727,8 +729,8 @@ __device__ inline float accept_limit(float tmax) {
 __device__ inline uint64_t lanes(bool b) { return __builtin_amdgcn_ballot_w64(b); }
 __device__ inline bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
-// STACK: the LDS stack's entries (kStack, or fewer for a smaller LDS
-// footprint and so more resident waves).  With STACK < kStack a ray that
+// STACK: the entries a ray may use (kStack or fewer; kRows of them stand in
+// LDS whatever it is).  With STACK < kStack a ray that
 // would push beyond it is abandoned and appended to the overflow list ovf
 // (ovf[0] the count, rays from ovf[1]); the caller traces those rays again
 // with kStack entries.  ray_list (optional): trace the rays ray_list[1 ..

@@ -119,11 +119,10 @@ class OnlineFineTune:
 
 class DynamicFrame:
     """Buffers and launch sequence of one frame of the dynamic scene.
-    primary_stack: LDS stack entries of the primary trace (16, 24 or 32;
-    rays that need more are traced again with 32 entries, so the records do
-    not change; coherent rays can gain from a short stack's extra resident
-    waves, the dynamic scene's measured none); the other traces use
-    config's stack.  concurrent_shadows: the shadow rays of each level are
+    primary_stack: stack entries of the primary trace (16, 24 or 32; rays
+    that need more are traced again with 32 entries, so the records do not
+    change, and the traversal keeps as many waves resident with any); the
+    other traces use config's stack.  concurrent_shadows: the shadow rays of each level are
     generated and traced on a second stream, beside the next bounce (both
     only read that level's hits), and an attached fine-tune stage runs on a
     third (it reads its level's rays and hits, the pair records and the
