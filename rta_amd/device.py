@@ -75,6 +75,21 @@ class DeviceBuffer:
             pass
 
 
+class DeviceView(DeviceBuffer):
+    """A part of an allocation, which it keeps alive and does not own."""
+
+    def __init__(self, owner: DeviceBuffer, offset: int, nbytes: int):
+        if offset < 0 or offset + nbytes > owner.nbytes:
+            raise ValueError("view exceeds the buffer")
+        self.owner, self.nbytes, self.ptr = owner, int(nbytes), owner.ptr + offset
+
+    def free(self) -> None:
+        self.owner, self.ptr = None, 0
+
+    def __del__(self):
+        pass
+
+
 class Stream:
     """A non-blocking HIP stream at default priority."""
 
