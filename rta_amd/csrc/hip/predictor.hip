@@ -20,6 +20,7 @@
 
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 namespace rta_hip {
@@ -511,14 +512,14 @@ __device__ inline v4f mfma32(v4u a, v4u b, v4f c) {
 
 // one 64-wide ReLU layer for NS sets of 16 rays; in: KS k-steps of B
 // operands per set, out: the next layer's 2 k-steps per set; record(k): the
-// lane's k-th weight record
-template <int KS, int NS, class Record>
+// lane's k-th weight record; bias(t): its four biases of row tile t
+template <int KS, int NS, class Record, class Bias>
 __device__ inline void hidden_layer(v4u out[NS][2], const v4u in[NS][KS], Record record,
-                                    const float *__restrict__ bias, int lane) {
+                                    Bias bias) {
 	unsigned d[NS][4][2];
 	#pragma unroll
 	for (int t = 0; t < 4; ++t) {
-		const float4 b = *reinterpret_cast<const float4 *>(bias + 16 * t + 4 * (lane >> 4));
+		const float4 b = bias(t);
 		v4f a[NS];
 		#pragma unroll
 		for (int r = 0; r < NS; ++r) a[r] = (v4f){b.x, b.y, b.z, b.w};
@@ -541,19 +542,35 @@ __device__ inline void hidden_layer(v4u out[NS][2], const v4u in[NS][KS], Record
 			out[r][s] = (v4u){d[r][2 * s][0], d[r][2 * s][1], d[r][2 * s + 1][0], d[r][2 * s + 1][1]};
 }
 
-// layer-1 B operands of the ray in lane column col (zero beyond n): octave
-// blocks 4s+g for s = 0..2 and the raw inputs (group 0) at s = 3
-__device__ inline void encode_operands(v4u x[4], const float *__restrict__ ro,
-                                       const float *__restrict__ rd, int ray, int n, float3 lo,
+// a ray's origin and direction (zero beyond n)
+struct RayInput {
+	float o[3], d[3];
+};
+
+__device__ inline RayInput load_ray(const float *__restrict__ ro, const float *__restrict__ rd,
+                                    int ray, int n) {
+	RayInput r = {};
+	if (ray < n)
+		#pragma unroll
+		for (int k = 0; k < 3; ++k) {
+			r.o[k] = ro[3 * (size_t)ray + k];
+			r.d[k] = rd[3 * (size_t)ray + k];
+		}
+	return r;
+}
+
+// layer-1 B operands of a ray (zero unless valid): octave blocks 4s+g for
+// s = 0..2 and the raw inputs (group 0) at s = 3
+__device__ inline void encode_operands(v4u x[4], const RayInput &r, bool valid, float3 lo,
                                        float3 scale, int g) {
 	float v0 = 0.f, v1 = 0.f, v2 = 0.f, v3 = 0.f, v4 = 0.f, v5 = 0.f;
-	if (ray < n) {
-		v0 = (ro[3 * (size_t)ray + 0] - lo.x) * scale.x - 1.0f;
-		v1 = (ro[3 * (size_t)ray + 1] - lo.y) * scale.y - 1.0f;
-		v2 = (ro[3 * (size_t)ray + 2] - lo.z) * scale.z - 1.0f;
-		v3 = rd[3 * (size_t)ray + 0];
-		v4 = rd[3 * (size_t)ray + 1];
-		v5 = rd[3 * (size_t)ray + 2];
+	if (valid) {
+		v0 = (r.o[0] - lo.x) * scale.x - 1.0f;
+		v1 = (r.o[1] - lo.y) * scale.y - 1.0f;
+		v2 = (r.o[2] - lo.z) * scale.z - 1.0f;
+		v3 = r.d[0];
+		v4 = r.d[1];
+		v5 = r.d[2];
 	}
 	// block 4s+g encodes input 2s + g/2, octaves 4*(g%2)..+3
 	const float in[3] = {(g & 2) ? v1 : v0, (g & 2) ? v3 : v2, (g & 2) ? v5 : v4};
@@ -616,7 +633,7 @@ __global__ __launch_bounds__(1024) void infer_kernel(const v4u *__restrict__ wp,
 	__shared__ v4u w4s[kRec4];
 	__shared__ v4f b4s[kOutP / 4];
 	__shared__ v4u w1s[8 * kWave], w23s[16 * kWave];
-	__shared__ float bs[3 * kHid];
+	__shared__ __attribute__((aligned(16))) float bs[3 * kHid];
 	for (int i = threadIdx.x; i < 8 * kWave; i += kInferWaves * kWave) {
 		w1s[i] = wp[pW1 + i];
 		w23s[i] = wp[pW2 + i];
@@ -651,10 +668,14 @@ __global__ __launch_bounds__(1024) void infer_kernel(const v4u *__restrict__ wp,
 	     tile += gridDim.x * kInferWaves) {
 		v4u x[2][4];
 		#pragma unroll
-		for (int r = 0; r < 2; ++r) encode_operands(x[r], ro, rd, tile * 32 + r * 16 + col, n, lo, scale, g);
-		// the hidden layers' weights and biases are loaded per tile: the empty asm hides their loop invariance, which would
-		// otherwise hoist all of them into registers and spill (an opaque
-		// offset, so that the loads stay global rather than flat)
+		for (int r = 0; r < 2; ++r) {
+			const int ray = tile * 32 + r * 16 + col;
+			encode_operands(x[r], load_ray(ro, rd, ray, n), ray < n, lo, scale, g);
+		}
+		// the hidden layers' weights and biases are loaded per tile: the
+		// empty asm hides their loop invariance, which would otherwise hoist
+		// all of them into registers and spill (an opaque offset, so that the
+		// loads keep their address spaces)
 		int z = 0;
 		asm volatile("" : "+s"(z));
 		const v4u *wq = wp + z;
@@ -663,9 +684,14 @@ __global__ __launch_bounds__(1024) void infer_kernel(const v4u *__restrict__ wp,
 		auto w1 = [&](int k) { return k < 8 ? w1s[z + k * kWave + lane] : wq[pW1 + k * kWave + lane]; };
 		auto w2 = [&](int k) { return w23s[z + k * kWave + lane]; };
 		auto w3 = [&](int k) { return w23s[z + (8 + k) * kWave + lane]; };
-		hidden_layer<4, 2>(h1, x, w1, bq, lane);
-		hidden_layer<2, 2>(h2, h1, w2, bq + kHid, lane);
-		hidden_layer<2, 2>(h3, h2, w3, bq + 2 * kHid, lane);
+		auto bias_of = [&](int layer) {
+			return [=](int t) {
+				return *reinterpret_cast<const float4 *>(bq + layer * kHid + 16 * t + 4 * g);
+			};
+		};
+		hidden_layer<4, 2>(h1, x, w1, bias_of(0));
+		hidden_layer<2, 2>(h2, h1, w2, bias_of(1));
+		hidden_layer<2, 2>(h3, h2, w3, bias_of(2));
 		float tk[2][4];
 		#pragma unroll
 		for (int r = 0; r < 2; ++r)
@@ -993,21 +1019,11 @@ __global__ __launch_bounds__(2 * SETS * kWave) void train_rows_kernel(
 	__shared__ float2 stat[SETS][2][16];
 	const int lane = __lane_id(), g = lane >> 4, col = lane & 15;
 	const int wave = (int)(threadIdx.x / kWave), sl = wave >> 1, half = wave & 1;
-	// W4's pack goes to LDS by direct global->LDS loads (64 records of 16 B
-	// per instruction, lane l's record at base + 16 l), all in flight while
-	// the first set's forward pass runs; waited for before its pass 1
-	for (int i = wave; i < kRec4 / 64; i += 2 * SETS)
-		__builtin_amdgcn_global_load_lds(
-		    (const __attribute__((address_space(1))) void *)(wp + pW4 + 64 * i + lane),
-		    (__attribute__((address_space(3))) void *)(w4s + 64 * i), 16, 0, 0);
-	for (int i = threadIdx.x; i < kOutP / 4; i += 2 * SETS * kWave)
-		b4s[i] = reinterpret_cast<const v4f *>(params + oB4)[i];
 	if (blockIdx.x == 0 && threadIdx.x == 0) *step += 1u;
 	uint16_t *t = tr[wave];
 	const int ld = out.ld;
-	// the loop runs the same number of times in every wave of the block, at
-	// least once (its barriers are reached by all of them)
-	for (int base = blockIdx.x * SETS; base < n_sets; base += gridDim.x * SETS) {
+	auto pass = [&](int base, auto first) {
+		constexpr bool FIRST = decltype(first)::value;
 		const int set = base + sl;
 		const bool act = set < n_sets;
 		const int ray0 = set * 16, ray = ray0 + col;
@@ -1020,15 +1036,50 @@ __global__ __launch_bounds__(2 * SETS * kWave) void train_rows_kernel(
 		asm volatile("" : "+s"(z));
 		const v4u *wq = wp + z;
 		const v4u *wqt = wpt + z;
-		v4u xs[1][4];
-		encode_operands(xs[0], ro, rd, act ? ray : n, n, lo, scale, g);
+		// everything the forward pass reads, in flight together, and with the
+		// first set W4's pack behind it by direct global->LDS loads (64 records
+		// of 16 B per instruction, lane l's record at base + 16 l): one memory
+		// latency at the start of the step instead of W4's, the rays' and each
+		// layer's in turn (32 steps of 8,192 rays 1,328 -> 1,298 us; 64 of 1,000
+		// 1,132 -> 1,110)
+		const RayInput in = load_ray(ro, rd, act ? ray : n, n);
 		const float *pq = params + z;
+		v4u wr[32];
+		float4 br[12];
+		#pragma unroll
+		for (int k = 0; k < 32; ++k)
+			wr[k] = wq[(k < 16 ? pW1 + k * kWave : k < 24 ? pW2 + (k - 16) * kWave : pW3 + (k - 24) * kWave) + lane];
+		#pragma unroll
+		for (int k = 0; k < 12; ++k)
+			br[k] = *reinterpret_cast<const float4 *>(pq + (k < 4 ? oB1 : k < 8 ? oB2 : oB3) + 16 * (k & 3) + 4 * g);
+		constexpr int kB4 = kOutP / 4, kThreads = 2 * SETS * kWave, kB4Rounds = (kB4 + kThreads - 1) / kThreads;
+		v4f b4r[kB4Rounds];
+		if (FIRST) {
+			#pragma unroll
+			for (int k = 0; k < kB4Rounds; ++k)
+				b4r[k] = reinterpret_cast<const v4f *>(params + oB4)[min((int)threadIdx.x + k * kThreads, kB4 - 1)];
+			__builtin_amdgcn_sched_barrier(0);
+			constexpr int kW4Loads = kRec4 / 64;
+			#pragma unroll
+			for (int k = 0; k < (kW4Loads + 2 * SETS - 1) / (2 * SETS); ++k) {
+				// (waves without a record in the last round load the last one)
+				const int i = min(k * 2 * SETS + wave, kW4Loads - 1);
+				__builtin_amdgcn_global_load_lds(
+				    (const __attribute__((address_space(1))) void *)(wp + pW4 + 64 * i + lane),
+				    (__attribute__((address_space(3))) void *)(w4s + 64 * i), 16, 0, 0);
+			}
+			__builtin_amdgcn_sched_barrier(0);
+		}
+		v4u xs[1][4];
+		encode_operands(xs[0], in, act && ray < n, lo, scale, g);
 		v4u h1[1][2], h2[1][2], h3[1][2];
-		const v4u *wq1 = wq + pW1, *wq2 = wq + pW2, *wq3 = wq + pW3;
-		hidden_layer<4, 1>(h1, xs, [&](int k) { return wq1[k * kWave + lane]; }, pq + oB1, lane);
-		hidden_layer<2, 1>(h2, h1, [&](int k) { return wq2[k * kWave + lane]; }, pq + oB2, lane);
-		hidden_layer<2, 1>(h3, h2, [&](int k) { return wq3[k * kWave + lane]; }, pq + oB3, lane);
-		if (base == blockIdx.x * SETS) {                  // W4 and its bias in LDS
+		hidden_layer<4, 1>(h1, xs, [&](int k) { return wr[k]; }, [&](int q) { return br[q]; });
+		hidden_layer<2, 1>(h2, h1, [&](int k) { return wr[16 + k]; }, [&](int q) { return br[4 + q]; });
+		hidden_layer<2, 1>(h3, h2, [&](int k) { return wr[24 + k]; }, [&](int q) { return br[8 + q]; });
+		if (FIRST) {                                      // W4 and its bias in LDS
+			#pragma unroll
+			for (int k = 0; k < kB4Rounds; ++k)
+				if ((int)threadIdx.x + k * kThreads < kB4) b4s[threadIdx.x + k * kThreads] = b4r[k];
 			__builtin_amdgcn_s_waitcnt(0);
 			__syncthreads();
 		}
@@ -1155,7 +1206,7 @@ __global__ __launch_bounds__(2 * SETS * kWave) void train_rows_kernel(
 		for (int off = kWave / 2; off > 0; off >>= 1) lossc += __shfl_xor(lossc, off);
 		if (act && lane == 0) out.loss_part[2 * set + half] = lossc * inv_m;
 		__syncthreads();
-		if (!act) continue;
+		if (!act) return;
 		if (half == 0) {
 			// the hidden layers' data gradients
 			#pragma unroll
@@ -1184,7 +1235,12 @@ __global__ __launch_bounds__(2 * SETS * kWave) void train_rows_kernel(
 			store_hidden(out.h2, ld, ray0, h2[0], t, lane);
 			store_hidden(out.h3, ld, ray0, h3[0], t, lane);
 		}
-	}
+	};
+	// every wave of the block makes the same passes, at least one (their
+	// barriers are reached by all of them)
+	pass(blockIdx.x * SETS, std::true_type{});
+	for (int base = (blockIdx.x + gridDim.x) * SETS; base < n_sets; base += gridDim.x * SETS)
+		pass(base, std::false_type{});
 }
 
 // dW and db of one layer for kGradNT row tiles of 16 (rows n0.., tiles at

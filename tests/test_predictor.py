@@ -396,6 +396,42 @@ def test_gradients_match_reference(gpu):
     assert np.all(g["W1"][:, 102:] == 0.0) and np.all(g["W4"][1025:] == 0.0)
 
 
+# 2 sets of 16 rays a block and, beyond 256 blocks' worth (8,192 rays), a
+# second pass of some blocks; padded to whole splits of 256 rays
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [17, 8192, 8193, 12000])
+def test_fused_step_gradients(gpu, n):
+    """The fused step's gradients and loss against the layered kernels', the
+    same network rounded to bf16 at the same points (activations, dOut, dZ),
+    so every one of three roundings on a path off by one unit bounds the
+    difference: 3 * 2^-8."""
+    o, d = _random_rays(n, 61)
+    rng = np.random.default_rng(62)
+    label = rng.integers(0, 1024, size=n).astype(np.int32)
+    label[rng.uniform(size=n) < 0.3] = -1
+    label[0] = 5
+    target = rng.normal(size=n).astype(np.float32)
+    ob, db = DeviceBuffer.from_array(o), DeviceBuffer.from_array(d)
+    lb, tb = DeviceBuffer.from_array(label), DeviceBuffer.from_array(target)
+    a = P.HitPredictor(16384, seed=19, scene_min=LO, scene_max=HI)
+    b = P.HitPredictor(16384, seed=19, scene_min=LO, scene_max=HI)
+    loss = DeviceBuffer(4)
+    loss.fill_u32(0)
+    call("rta_pred_zero_grads", a.h, None)
+    a.forward(ob, db, n)
+    call("rta_pred_backward", a.h, ptr(lb), ptr(tb), n, ptr(loss), None)
+    b.loss.fill_u32(0)
+    b.train_step(ob, db, lb, tb, n)
+    rta_amd.synchronize()
+    la, lf = float(loss.download(np.float32, 1)[0]), float(b.loss.download(np.float32, 1)[0])
+    assert abs(la - lf) < 3 * 2.0 ** -8 * abs(la)
+    ga, gf = P.unpack(a.grads()), P.unpack(b.grads())
+    for name in ga:
+        err = np.linalg.norm(gf[name] - ga[name]) / np.linalg.norm(ga[name])
+        say(f"{n} rays, {name}: {err:.1e}")
+        assert err < 3 * 2.0 ** -8, name
+
+
 # ------------------------------------------------------------- treelets
 
 def cut_restatement(nodes, ranges, n, max_treelets):
