@@ -784,6 +784,9 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 	const int quad = lane & 3;
 	// byte b (a multiple of 8) of this lane's record in the stage
 	LdsByte *const record = (LdsByte *)&stage[wave][quad][lane & ~3];
+	// the staged fetch puts a quarter's number into the low bits of its record's
+	// address; records that are not 64-byte aligned are gathered
+	const int stage_min = ((uintptr_t)pairs & 63u) == 0 ? kStageMin : kWave + 1;
 	auto staged = [&](int b) { return (const LdsPair *)(record + ((((b >> 4) ^ quad) << 4) | (b & 8))); };
 
 	uint32_t curr = kIdle, top = kIdle, ray = kNoRay;
@@ -1182,7 +1185,7 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 		// Lanes whose neighbour stands at another node: coherent waves gather
 		const uint32_t beside = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)curr, 0xb1, 0xf, 0xf, true);
 		const int apart = __popcll(lanes((curr & 1u) != 0u && beside != curr));
-		if (apart < kStageMin)
+		if (apart < stage_min)
 			run(std::true_type{});
 		else
 			run(std::false_type{});
