@@ -50,13 +50,16 @@ __global__ __launch_bounds__(256) void morton_kernel(
 // rs_scatter_kernel does), four threads per digit turn the counts over (item,
 // wave) -- index order -- into positions, and the keys move through LDS.
 //
-// What bounds it: latency and the issue rate of one CU.  It replaces fourteen
-// launches of 3 to 8 us each.  Whole builds, before and after: 1,000
-// triangles 66 -> 37 us, 4,096 100 -> 62, 8,192 105 -> 82, 12,288 107 -> 100;
-// larger meshes take the launches (14,000 triangles: 108 us).
+// What bounds it: latency and the issue rate of one CU.  It replaces eight
+// launches (bounds, codes, three sort passes of two kernels).  Whole packed
+// builds, with those launches and with this kernel: 1,024 triangles 55 and 37
+// us, 2,048 67 and 52, 4,096 72 and 63, 5,120 73 and 71, 6,144 74 and 73;
+// larger meshes take the launches (7,168: 76 and 82, 8,192 76 and 84, 12,288
+// 81 and 103).  A build that is waited for crosses a little higher, as its
+// launches are not hidden: 6,145 triangles 100 and 95 us, 8,192 97 and 98.
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallWaves = kSmallThreads / kWave;
-constexpr int kSmallItems = 12;   // 16 would not fit in registers
+constexpr int kSmallItems = 6;
 constexpr int kSmallSort = kSmallItems * kSmallThreads;
 
 template <int K>
@@ -437,9 +440,6 @@ static int small_sort(uint32_t *indices, const LbvhWorkspace &w, uint32_t *statu
 	if (items <= 1) launch(small_sort_kernel<1>);
 	else if (items <= 2) launch(small_sort_kernel<2>);
 	else if (items <= 4) launch(small_sort_kernel<4>);
-	else if (items <= 6) launch(small_sort_kernel<6>);
-	else if (items <= 8) launch(small_sort_kernel<8>);
-	else if (items <= 10) launch(small_sort_kernel<10>);
 	else launch(small_sort_kernel<kSmallItems>);
 	RTA_LAUNCH_CHECK("small_sort_kernel");
 	return RTA_OK;
