@@ -616,7 +616,7 @@ __device__ inline int key_cluster(float k) { return 1023 - (int)(__float_as_uint
 // a ray's top are written as -1).
 //
 // A tile whose logits could overflow to infinity (`wild`: a weight, bias or
-// activation of layer 4 beyond 2^34, 2^66 or 2^65) inserts its keys one by
+// activation of layer 4 from 2^34, 2^66 or 2^66 on) inserts its keys one by
 // one, in treelet order: such keys are NaNs and their order matters.  So do
 // top-4 launches of at most one wave a SIMD, which wait for the four-key
 // checks' branches (2,000 rays 18.6 us with the checks, 15.4 without; 30,000
