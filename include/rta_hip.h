@@ -69,7 +69,10 @@ typedef struct __attribute__((aligned(64))) rta_node_pair {
 
 /* Per-stage build times in milliseconds (hipEvent based), in the stage
  * order of bbvh-cuda/lbvh.h:173-198.  The hierarchy is emitted by the
- * bottom-up pass, so `tree` is (close to) zero and `boxes` covers both. */
+ * bottom-up pass, so `tree` is (close to) zero and `boxes` covers both.  Up
+ * to 6,144 triangles one kernel forms the scene box, the codes and their
+ * order, so `voxel_bounds` and `morton` are (close to) zero and `sort` covers
+ * the three. */
 typedef struct rta_lbvh_times {
 	float init_triangles, voxel_bounds, morton, sort, tree, boxes, permute;
 	float total;

@@ -1040,7 +1040,7 @@ __global__ __launch_bounds__(2 * SETS * kWave) void train_rows_kernel(
 		// first set W4's pack behind it by direct global->LDS loads (64 records
 		// of 16 B per instruction, lane l's record at base + 16 l): one memory
 		// latency at the start of the step instead of W4's, the rays' and each
-		// layer's in turn (32 steps of 8,192 rays 1,328 -> 1,298 us; 64 of 1,000
+		// layer's in turn (32 steps of 8,192 rays 1,328 -> 1,298 us; 33 of 1,000
 		// 1,132 -> 1,110)
 		const RayInput in = load_ray(ro, rd, act ? ray : n, n);
 		const float *pq = params + z;

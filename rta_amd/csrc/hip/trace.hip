@@ -677,7 +677,9 @@ constexpr int kRows = 11, kSpill = 5;
 // 2.3 M-triangle terrain).  A wave claims a slot in the bitmap at its first
 // spill and gives it back when it ends.  LDS holds 21 of these waves per CU,
 // so 8,192 slots are never all taken by the waves of 256 CUs; a wave that
-// finds none counts a stack overflow.  Private memory would do, but a
+// finds none counts a stack overflow.  The entries (52.4 MB on each GPU) are
+// there from the module's load on, about 20 ms of it, once per process.
+// Private memory would do, but a
 // queue's first launch with scratch allocates it for the whole machine (0.3
 // to 1.1 ms on each new stream).
 //
@@ -752,9 +754,9 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 	// them the bottom mark kIdle; `sp` points at the last of those rows (row
 	// 0 while there is none).  Row 0 is read, and its value dropped, when a
 	// lane pops the mark (sp is row -1 from then on; the idle lane may still
-	// read there, and write row 0); row kRows + 1 is written when a lane whose rows are
-	// full takes a step.  A push beyond kRows first moves the lowest kSpill
-	// rows (or what is left of STACK) to the wave's deep slot, `spilled`
+	// read there, and write row 0); row kRows + 1 is written when a lane whose
+	// rows are full takes a step.  A push beyond kRows first moves the lowest
+	// kSpill rows (or what is left of STACK) to the wave's deep slot, `spilled`
 	// entries of this lane.
 	__shared__ uint32_t stack[(kRows + 3) * BLOCK];
 	__shared__ float4 stage[BLOCK / kWave][4][kWave];   // see run
@@ -795,11 +797,13 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 	// one atomic: what it needs now or, if more, a share of what is left.
 	// The queue is one word whose atomics take turns (about 7 ns each), which
 	// bounded launches of short rays when every refill took one: 64 meshes'
-	// build and 4.45 M-ray trace 1,922 us, with shares of 1/4, 1/2 and 1/1 of
-	// an even split 1,688 / 1,584 / 1,613 us.  Long rays lose to uneven ends
-	// what larger shares save (primary rays of the 2.3 M-triangle terrain
-	// 1,621 us, then 1,623 / 1,661 / 1,963; bounce rays 1,568, then 1,551 /
-	// 1,539 / 1,694), so one mesh takes 1/4 and a batch 1/2.
+	// build and 4.45 M-ray trace 1,922 us, with `split` 4, 2 and 1 times the
+	// waves 1,688 / 1,584 / 1,613 us.  (The share is what is left over the next
+	// power of two above split: for 5,120 waves 1/6.4, 1/3.2 and 1/1.6 of an
+	// even split.)  Long rays lose to uneven ends what larger shares save
+	// (primary rays of the 2.3 M-triangle terrain 1,621 us, then 1,623 / 1,661 /
+	// 1,963; bounce rays 1,568, then 1,551 / 1,539 / 1,694), so one mesh takes 4
+	// and a batch 2.
 	uint32_t run_at = 0, run_end = 0, left = n;
 	// With fixed_rays the wave's only run is its own, without the queue.
 	if (fixed_rays) {
