@@ -666,10 +666,11 @@ typedef __attribute__((address_space(3))) Pair LdsPair;
 typedef __attribute__((address_space(1))) char GlobalByte;
 // Stack rows in LDS, and how many of them move to device memory at once.
 // With the 4 KiB stage, 11 + 3 rows make 7,680 B per wave, six of the 1,280-B
-// units LDS is handed out in: 20 resident waves per CU, where 13 rows leave
-// 18 (primary rays 1,634 against 1,688 us, bounce rays 1,582 against 1,602 us
-// per 2.07 M on the 2.3 M-triangle terrain); 9 rows spill more and gain no
-// wave (1,659 / 1,607 us).
+// units LDS is handed out in: 21 resident waves per CU (20 for a batch, whose
+// registers allow five a SIMD).  With 20 waves, 13 rows (18 waves) took 1,688
+// us against 1,634 for primary and 1,602 against 1,582 us for bounce rays (2.07
+// M on the 2.3 M-triangle terrain); 9 rows spill more and gained no wave
+// (1,659 / 1,607 us).
 constexpr int kRows = 11, kSpill = 5;
 
 // Where they move to: slots of kDeep entries per lane, one per wave that

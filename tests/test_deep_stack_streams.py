@@ -18,7 +18,7 @@ from test_short_stack import Packed, same_records
 from test_traversal_paths import forest, forest_rays
 
 ROUNDS = 12
-RAYS = 163841            # 64 a wave: 2,561 waves, nearly all with deep rays
+RAYS = 200001            # 64 a wave: 3,126 waves, nearly all with deep rays
 
 
 @pytest.mark.gpu

@@ -16,7 +16,7 @@ from rta_amd.device import DeviceBuffer
 from test_short_stack import Packed, same_records
 
 BASE = 4096
-WHOLE_WAVES = 163841      # more rays than 5,120 resident waves take by halves
+WHOLE_WAVES = 200001      # more than 24 waves on each of 256 CUs take by halves
 
 
 def mesh(flagged: bool):
