@@ -666,12 +666,17 @@ typedef __attribute__((address_space(3))) Pair LdsPair;
 typedef __attribute__((address_space(1))) char GlobalByte;
 // Stack rows in LDS, and how many of them move to device memory at once.
 // With the 4 KiB stage, 11 + 3 rows make 7,680 B per wave, six of the 1,280-B
-// units LDS is handed out in: 21 resident waves per CU (20 for a batch, whose
-// registers allow five a SIMD).  With 20 waves, 13 rows (18 waves) took 1,688
-// us against 1,634 for primary and 1,602 against 1,582 us for bounce rays (2.07
-// M on the 2.3 M-triangle terrain); 9 rows spill more and gained no wave
-// (1,659 / 1,607 us).
+// units LDS is handed out in: 20 resident waves per CU, where 13 rows leave
+// 18 (primary rays 1,634 against 1,688 us, bounce rays 1,582 against 1,602 us
+// per 2.07 M on the 2.3 M-triangle terrain); 9 rows spill more and gain no
+// wave (1,659 / 1,607 us).
 constexpr int kRows = 11, kSpill = 5;
+// Waves per CU of a launch: five a SIMD.  LDS and registers would hold a 21st,
+// which gains on large scenes (the rays above 1,588 against 1,610 us and 1,540
+// against 1,550) and loses where two launches run at once (frames of 14
+// k-triangle scenes at 3537 x 1874 3,110 against 3,074 us, of 270 k at 1564 x
+// 752 1,302 against 1,282).
+constexpr int kWavesPerCu = 20;
 
 // Where they move to: slots of kDeep entries per lane, one per wave that
 // needs any (rays deeper than 11 entries: 0.4 % of the bounce rays of a
@@ -865,8 +870,8 @@ __global__ __launch_bounds__(BLOCK, 5) void trace_cis_persistent_kernel(
 	// division-free one, on the record that the step has fetched anyway: where
 	// every lane took the latter and slow ones then loaded their record again,
 	// 2 M rays of the 2.3 M-triangle terrain took 1,881 us straight down (now
-	// 1,509), 2,440 us parallel to a plane in no order (1,793) and 2,205 us with
-	// one such ray in 16 (2,028).
+	// 1,515), 2,440 us parallel to a plane in no order (1,816) and 2,205 us with
+	// one such ray in 16 (2,032).
 	auto ieee_slabs = [&](const float4 &q0, const float4 &q1, const float4 &q2, float &dl, float &fl,
 	                      float &dr, float &fr) {
 		bool hl, hr;
@@ -1380,7 +1385,7 @@ int launch_persistent(const float *tri4, const rta_node_pair *pairs, const uint3
 		RTA_HIP_TRY(hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev));
 		RTA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(
 		    &o, trace_cis_persistent_kernel<BLOCK, ANY_HIT, BATCHED, SEEDED, STACK>, BLOCK, 0));
-		occ[dev] = o < 1 ? 1 : o;
+		occ[dev] = std::min(std::max(o, 1), kWavesPerCu * kWave / BLOCK);
 		cus[dev] = c;
 	}
 	const int bpc = blocks_per_cu > 0 ? blocks_per_cu : occ[dev];
