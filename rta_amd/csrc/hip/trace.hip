@@ -630,7 +630,7 @@ __global__ void fill_queue_kernel(uint32_t *queue) {
 // staged fetch in `run` below; coherent rays the VALU (about 95
 // instructions per wave-step at inner nodes, 116 before the stack's top
 // moved to a register, the decision's masks to scalar registers and the
-// records' stores out of the step; 96 % of the issue slots, 81 % for bounce
+// records' stores out of the step; 95 % of the issue slots, 82 % for bounce
 // rays).  On the 2.3 M-triangle terrain, 2.07 M rays each: bounce rays 1,910
 // -> 1,549 us, primary rays 1,890 -> 1,636 us; shadow rays of a 400
 // k-triangle terrain (0.88 M) 750 -> 640 us.
